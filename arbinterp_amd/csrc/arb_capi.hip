@@ -184,7 +184,6 @@ struct arb_field {
     void* table = nullptr;      // [nc+1][ninterp][K]: FP64 or FP32, allocated on first build
     int64_t table_bytes = 0;
     void* sent = nullptr;       // [ninterp][K] the sentinel row, for paths without the table
-    double* A = nullptr;        // K x K FP64
     int32_t* flag = nullptr;    // device status word
     // bucketed query path: block geometry of the table kernels (B) and of the
     // fused kernel (BF, without the larger blocks that only save a sort pass)
@@ -217,11 +216,11 @@ struct arb_field {
     int32_t* bw_hist = nullptr;    // its tile histograms (256 per tile)
     int32_t* bw_hscan = nullptr;   // and their scans (+ 256 digit totals)
     double* bw_part = nullptr;     // sums of chunks of cells holding many queries
-    double* bw_rec = nullptr;      // 3D: per query u, v, w, gv, gg / h (8 doubles)
+    double* bw_rec = nullptr;      // per query: local coordinates, gv, gg / h
     int64_t bw_n = 0;
     int32_t* bw_count = nullptr;   // the radix sort's first positions
     int32_t* bw_offs = nullptr;    // nc + 1
-    double* bw_bbar = nullptr;     // node-adjoint scratch: 3D block tiles, 4D K x nc
+    double* bw_bbar = nullptr;     // node-adjoint scratch: the blocks' node tiles
     // particle push graph
     hipStream_t cap_stream = nullptr;
     hipGraphExec_t push_exec = nullptr;
@@ -563,14 +562,8 @@ int arb_field_create(const double* rows_dev, int64_t nrows, int32_t ncols, int64
     HIPCHK(hipStreamSynchronize(s));
     if (hflag) return fail(ARB_EGRID, "rows do not form a complete grid (duplicate points)");
 
-    // 4. operator matrix and table storage
+    // 4. table size and the sentinel row
     const int K = 1 << (2 * ndim);
-    std::vector<double> Bi, D, A;
-    make_invB(ndim, Bi);
-    make_D(ndim, D);
-    matmul(K, Bi, D, A);
-    HIPCHK(hipMalloc(&f->A, sizeof(double) * K * K));
-    HIPCHK(hipMemcpyAsync(f->A, A.data(), sizeof(double) * K * K, hipMemcpyHostToDevice, s));
     const size_t esz = precision == ARB_PREC_FP64 ? sizeof(double) : sizeof(float);
     // the table itself is allocated by its first build (node-tile queries
     // never read it)
@@ -1234,7 +1227,7 @@ int arb_query_backward(arb_field* f, const double* q_dev, int64_t n, int64_t ldq
             HIPCHK(hipMalloc(&f->bw_hist, sizeof(int32_t) * hl));
             HIPCHK(hipMalloc(&f->bw_hscan, sizeof(int32_t) * (hl + 256)));
             HIPCHK(hipMalloc(&f->bw_part, sizeof(double) * arb_bwd_part_elems(f->g, m)));
-            if (f->g.ndim == 3) HIPCHK(hipMalloc(&f->bw_rec, sizeof(double) * 8 * m));
+            HIPCHK(hipMalloc(&f->bw_rec, sizeof(double) * arb_bwd_rec_elems(f->g) * m));
             f->bw_n = n;
         }
         if (!f->bw_bbar) {
@@ -1252,8 +1245,8 @@ int arb_query_backward(arb_field* f, const double* q_dev, int64_t n, int64_t ldq
     // same tiles) and writes each query's record at its grouped position.
     // From the 3D table (a cell's 64 coefficients one contiguous 512-byte
     // read), in query order, with the keys and records by row.  From the
-    // 4D table (2 KB per cell), in the grouped order again; 4D has no
-    // records.
+    // 4D table (2 KB per cell), in the grouped order again, with the records
+    // at the grouped positions.
     const bool grouped = dval_dev && nodes;
     const bool grouped4 = dval_dev && !nodes && f->g.ndim == 4;
     if ((grouped || grouped4) && n > 0)
@@ -1283,11 +1276,10 @@ int arb_query_backward(arb_field* f, const double* q_dev, int64_t n, int64_t ldq
     if (n > 0 && grouped4)
         HIPCHK(arb_launch_bwd_points(f->g, f->precision, f->table, f->ninterp, f->ninterp - 1,
                                      q_dev, n, ldq, gv_dev, gg_dev, dq_dev, perm, nullptr,
-                                     nullptr, s));
+                                     f->bw_rec, s));
     if (dval_dev) {
-        HIPCHK(arb_launch_bwd_cells(f->g, f->A, q_dev, ldq, gv_dev, gg_dev, f->bw_rec,
-                                    grouped ? 1 : 0, f->bw_offs, perm, n, f->bw_part, f->bw_bbar,
-                                    s));
+        HIPCHK(arb_launch_bwd_cells(f->g, q_dev, ldq, f->bw_rec, grouped ? 1 : 0, f->bw_offs, perm,
+                                    n, f->bw_part, f->bw_bbar, s));
         HIPCHK(arb_launch_bwd_nodes(f->g, f->bw_bbar, dval_dev, s));
     }
     return ARB_OK;
@@ -1605,7 +1597,6 @@ void arb_field_destroy(arb_field* f) {
     if (f->tiles) (void)hipFree(f->tiles);
     if (f->table) (void)hipFree(f->table);
     if (f->sent) (void)hipFree(f->sent);
-    if (f->A) (void)hipFree(f->A);
     if (f->flag) (void)hipFree(f->flag);
     if (f->ws_bkt) (void)hipFree(f->ws_bkt);
     if (f->ws_rank) (void)hipFree(f->ws_rank);

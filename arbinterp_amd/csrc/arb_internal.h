@@ -372,7 +372,8 @@ hipError_t arb_launch_eval_perm(const ArbGeom& g, const ArbBuckets& B, int32_t p
 hipError_t arb_launch_bwd_keys(const ArbGeom& g, const double* q, int64_t n, int64_t ldq,
                                int32_t* key, hipStream_t s);
 // Backward of interpolant kn from the table: d/dq, and for the node adjoint
-// (key, rec non-null) the query's cell key and (3D) its record at row i.
+// (key, rec non-null) the query's cell key and its record (3D: at row i; 4D:
+// at the grouped position).
 // perm (or nullptr): the queries in grouped order; thread s then takes
 // query perm[s].
 hipError_t arb_launch_bwd_points(const ArbGeom& g, int32_t prec, const void* table,
@@ -383,10 +384,11 @@ hipError_t arb_launch_bwd_points(const ArbGeom& g, int32_t prec, const void* tab
 // part: arb_bwd_part_elems(g, n) doubles of scratch (the sums of chunks of
 // cells holding many queries).
 int64_t arb_bwd_part_elems(const ArbGeom& g, int64_t n);
+// Doubles of a query's record (3D, 4D).
+int64_t arb_bwd_rec_elems(const ArbGeom& g);
 // rec_grouped: the 3D records sit at the queries' grouped positions (else by
-// row, reached through perm).
-hipError_t arb_launch_bwd_cells(const ArbGeom& g, const double* A, const double* q, int64_t ldq,
-                                const double* gv, const double* gg, const double* rec,
+// row, reached through perm); the 4D ones always do.
+hipError_t arb_launch_bwd_cells(const ArbGeom& g, const double* q, int64_t ldq, const double* rec,
                                 int32_t rec_grouped, const int32_t* offs, const int32_t* perm,
                                 int64_t n, double* part, double* bbar, hipStream_t s);
 hipError_t arb_launch_bwd_nodes(const ArbGeom& g, const double* bbar, double* dval, hipStream_t s);

@@ -7,39 +7,22 @@
 //            c_i = gv_i m(x_i) + sum_k gg_ik dm_k(x_i)/h_k
 // The node adjoint is deterministic: queries are grouped per cell in
 // query-index order (a stable radix sort of the cell keys, k_sort.hip), and
-// the per-cell 64 (256)-vector alpha_bar is summed in that order.  3D: the
-// per-query records are written by row (table path) or, from the node
-// tiles, at the queries' grouped positions (a cell's records consecutive).  3D: blocks of 4^3
-// cells apply the transpose of the separable coefficient passes to their
-// alpha_bar, giving partial gradients on the block's 7^3 node tile, and
-// every node sums the tiles holding it in a fixed block order.  4D:
-// b_bar = A^T alpha_bar per cell, stored slot-major bbar[l][cell], and every
-// node gathers b_bar from its <= 4^4 cells in a fixed slot order.  No
-// floating-point atomics.
+// every per-cell sum runs in that order over per-query records, written by
+// row (3D table path) or at the queries' grouped positions (node tiles and
+// 4D: a cell's records consecutive).  3D: blocks of 4^3 cells apply the
+// transpose of the separable coefficient passes to their alpha_bar, giving
+// partial gradients on the block's 7^3 node tile, and every node sums the
+// tiles holding it in a fixed block order.  4D does the same with blocks of
+// 4 x 4 x 2 cells in (x, y, z) that run through all of t (k_bwd_block4), the
+// operator's row shift included.  No floating-point atomics.
 #include "arb_internal.h"
 
 namespace {
-
-template <int D>
-struct Basis1 {
-    double b0[D][4], b1[D][4], b2[D][4];
-};
 
 // t[e] for a runtime e in 0..3 by selects (a dynamic index into a register
 // array would place the array in scratch memory)
 __device__ __forceinline__ double sel4(const double* t, int e) {
     return e == 0 ? t[0] : e == 1 ? t[1] : e == 2 ? t[2] : t[3];
-}
-
-template <int D>
-__device__ __forceinline__ void make_basis(const double* loc, Basis1<D>& B) {
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-        const double u = loc[a];
-        B.b0[a][0] = 1.0; B.b0[a][1] = u; B.b0[a][2] = u * u; B.b0[a][3] = u * u * u;
-        B.b1[a][0] = 0.0; B.b1[a][1] = 1.0; B.b1[a][2] = 2.0 * u; B.b1[a][3] = 3.0 * u * u;
-        B.b2[a][0] = 0.0; B.b2[a][1] = 0.0; B.b2[a][2] = 2.0; B.b2[a][3] = 6.0 * u;
-    }
 }
 
 // p(u), p'(u) and p''(u)/2 of c0 + c1 u + c2 u^2 + c3 u^3 (synthetic division).
@@ -132,13 +115,17 @@ k_bwd_keys(ArbGeom g, const double* __restrict__ q, int64_t n, int64_t ldq,
     key[i] = flat < g.nc ? (int32_t)flat : (int32_t)g.nc;
 }
 
-// d/dq per query, and, for the node adjoint, the query's cell key and (3D)
-// its record at row i.  Without perm, thread i takes query i: 3D reads a
-// cell's 64 table coefficients as one contiguous 512-byte run, so query
-// order costs nothing and the queries' own arrays are read and written in
-// order.  With perm (the queries grouped by cell; 4D, whose 256
-// coefficients of a cell are 2 KB), thread s takes query perm[s], so
-// neighbouring threads read the same cell's coefficients.
+// Doubles of a 4D record: u, v, w, t, gv, gg / h (4), one of padding (16-byte
+// loads).
+constexpr int REC4 = 10;
+
+// d/dq per query, and, for the node adjoint, the query's cell key and its
+// record (3D: at row i; 4D: at the grouped position s).  Without perm,
+// thread i takes query i: 3D reads a cell's 64 table coefficients as one
+// contiguous 512-byte run, so query order costs nothing and the queries' own
+// arrays are read and written in order.  With perm (the queries grouped by
+// cell; 4D, whose 256 coefficients of a cell are 2 KB), thread s takes query
+// perm[s], so neighbouring threads read the same cell's coefficients.
 template <int D, typename TC>
 __global__ void __launch_bounds__(256)
 k_bwd_points(ArbGeom g, const TC* __restrict__ table, int32_t ninterp, int32_t kn,
@@ -158,9 +145,18 @@ k_bwd_points(ArbGeom g, const TC* __restrict__ table, int32_t ninterp, int32_t k
     if (key) key[i] = ok ? (int32_t)flat : (int32_t)g.nc;  // rows outside: after the cells
     if (rec && ok) {
         // the node adjoint's per-query record: local coordinates, gv, gg / h
-        double4* r4 = reinterpret_cast<double4*>(rec + i * 8);
-        r4[0] = make_double4(loc[0], loc[1], loc[2], gv[i]);
-        r4[1] = make_double4(gg[i * 3] / g.h[0], gg[i * 3 + 1] / g.h[1], gg[i * 3 + 2] / g.h[2], 0.0);
+        if constexpr (D == 3) {
+            double4* r4 = reinterpret_cast<double4*>(rec + i * 8);
+            r4[0] = make_double4(loc[0], loc[1], loc[2], gv[i]);
+            r4[1] = make_double4(gg[i * 3] / g.h[0], gg[i * 3 + 1] / g.h[1], gg[i * 3 + 2] / g.h[2], 0.0);
+        } else {
+            double2* r2 = reinterpret_cast<double2*>(rec + s * REC4);
+            r2[0] = make_double2(loc[0], loc[1]);
+            r2[1] = make_double2(loc[2], loc[3]);
+            r2[2] = make_double2(gv[i], gg[i * 4] / g.h[0]);
+            r2[3] = make_double2(gg[i * 4 + 1] / g.h[1], gg[i * 4 + 2] / g.h[2]);
+            r2[4] = make_double2(gg[i * 4 + 3] / g.h[3], 0.0);
+        }
     }
     if (!dq) return;
     if (!ok) {
@@ -179,46 +175,6 @@ k_bwd_points(ArbGeom g, const TC* __restrict__ table, int32_t ninterp, int32_t k
 #pragma unroll
         for (int y = 0; y < D; ++y) acc += (H[x][y] / (g.h[x] * g.h[y])) * gg[i * D + y];
         dq[i * D + x] = acc;
-    }
-}
-
-// alpha_bar[j] of one 4D cell for the entries j = j0 + 64 r (r < 4; j0 a
-// lane): the sum over the cell's queries, in query-index order, of
-// gv m_j + sum_x gk_x dm_j/dx.  With j = e0 + 4 e1 + 16 e2 + 64 e3, lane j0
-// fixes e0, e1, e2 and r is e3, so m_j = P b0_t[r] with P = u^e0 v^e1 w^e2
-// shared by the lane's four entries:
-//   t_j = (gv P + gk_u P_u + gk_v P_v + gk_w P_w) b0_t[r] + gk_t P b1_t[r].
-template <int D, int R>
-__device__ __forceinline__ void cell_abar(const ArbGeom& g, const double* __restrict__ q,
-                                          int64_t ldq, const double* __restrict__ gv,
-                                          const double* __restrict__ gg, const int32_t* perm,
-                                          int32_t s0, int32_t s1, int j0, int stride,
-                                          double* acc) {
-    static_assert(D == 4 && R == 4, "4D: lane j0 holds the entries j0 + 64 r");
-    (void)stride;
-#pragma unroll
-    for (int r = 0; r < R; ++r) acc[r] = 0.0;
-    const int e0 = j0 & 3, e1 = (j0 >> 2) & 3, e2 = (j0 >> 4) & 3;
-    for (int32_t s = s0; s < s1; ++s) {
-        const int64_t i = perm[s];
-        double loc[D];
-        bool oob;
-        (void)arb_reduce<D>(q + i * ldq, g, loc, &oob);
-        Basis1<D> B;
-        make_basis<D>(loc, B);
-        const double v = gv[i];
-        double gk[D];
-#pragma unroll
-        for (int x = 0; x < D; ++x) gk[x] = gg[i * D + x] / g.h[x];
-        const double a0 = sel4(B.b0[0], e0), a1 = sel4(B.b0[1], e1), a2 = sel4(B.b0[2], e2);
-        const double d0 = sel4(B.b1[0], e0), d1 = sel4(B.b1[1], e1), d2 = sel4(B.b1[2], e2);
-        const double a01 = a0 * a1;
-        const double P = a01 * a2;
-        const double Pu = d0 * a1 * a2, Pv = a0 * d1 * a2, Pw = a01 * d2;
-        const double c = v * P + gk[0] * Pu + gk[1] * Pv + gk[2] * Pw;
-        const double e = gk[3] * P;
-#pragma unroll
-        for (int r = 0; r < R; ++r) acc[r] += c * B.b0[3][r] + e * B.b1[3][r];
     }
 }
 
@@ -475,122 +431,345 @@ k_bwd_nodes3(ArbGeom g, const double* __restrict__ tiles, int64_t nbx, int64_t n
     dval[nidx] = sum;
 }
 
-// 4D: a workgroup per 16 cells: one wave per cell at a time sums alpha_bar
-// (256) over the cell's queries in index order, then b_bar = A^T alpha_bar
-// for the 16 cells together (each element of A read once per workgroup),
-// written slot-major bbar[l][cell].
-// 4D chunk sums (cells of more than BWD_CHUNK queries): one wave per chunk,
-// part[o][entry] (256 entries).
-template <int D>
-__global__ void __launch_bounds__(256)
-k_bwd_chunk(ArbGeom g, const double* __restrict__ q, int64_t ldq, const double* __restrict__ gv,
-            const double* __restrict__ gg, const int32_t* __restrict__ offs,
-            const int32_t* __restrict__ perm, int64_t nchunk, double* __restrict__ part) {
-    constexpr int K = 1 << (2 * D);
-    constexpr int PER = K / 64;
-    const int lane = threadIdx.x & 63;
-    const int64_t o = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    int32_t s0, s1;
-    if (o >= nchunk || !bwd_chunk<D>(g, q, ldq, offs, perm, o, &s0, &s1)) return;
-    double acc[PER];
-    cell_abar<D, PER>(g, q, ldq, gv, gg, perm, s0, s1, lane, 64, acc);
+// 4D node adjoint.  alpha = (M (x) M (x) M (x) M) F + P c with alpha_85 = 0
+// (arb_sep4.h): c_k = G(k-1) - G(k), G the xyzt central difference at the
+// cell's corner nodes.  Its transpose, per cell:
+//   alpha_bar_85 = 0;  c_bar = P^T alpha_bar;  G_bar(j) = c_bar_{j+1} - c_bar_j;
+//   F_bar = (M (x) M (x) M (x) M)^T alpha_bar + the transposed differences of G_bar.
+// The central difference at an end of the cell is the derivative of the
+// cell's cubic there, a_1 at u = 0 and a_1 + 2 a_2 + 3 a_3 at u = 1, so the
+// last term is (M (x) ..)^T of X (x) X (x) X (x) X G_bar with X = [[0,0], [1,1],
+// [0,2], [0,3]] (power x end), and one transposed separable pass serves both.
+//
+// A workgroup takes a block of 4 x 4 x 2 cells in (x, y, z) and runs through
+// all of t.  Eight threads per cell: thread gq holds, for the (ex, ey) pairs
+// 2 gq and 2 gq + 1, the four ez and the four t planes that the cell touches,
+//   ring[ot][pair][ez] = sum over queries of Q(ex, ey, ez) w_ot(t) + E w'_ot(t),
+// w_ot the node weights along t (M applied to the powers of t, so the t pass
+// is done query by query), Q = gv m + gk_u m_u + gk_v m_v + gk_w m_w and E = gk_t m
+// for the monomial m = u^ex v^ey w^ez; and c_bar of the corners gq and gq + 8,
+// from the Hermite end weights h_0 = t - 2t^2 + t^3, h_1 = t^3 - t^2 (the columns of
+// P).  After cell layer ct, plane ct is complete: it goes through the
+// transposed z, y and x passes to the block's 7 x 7 x 5 nodes of that plane,
+// tiles[block][plane][node], and the ring moves on by one.  So a cell costs
+// about 160 FP64 operations per query and thread, the passes run once per
+// node plane instead of once per cell layer and power of t, and 9 doubles
+// per cell go to memory.  On 48^3 x 16 nodes, 2e6 queries: 0.61 ms; A^T
+// alpha_bar per cell (65536 products a cell, 256 doubles of it written and
+// gathered) took 7.5 ms.  The node sums: 0.03 beside 0.62 ms.  It is bound by
+// FP64 issue and the latency of offs -> record at two waves per SIMD (250
+// VGPRs); sixteen threads per cell and 4 x 4 x 1 cells run four waves, but
+// repeat more of each query's work: 0.69 ms.
+constexpr int B4X = 4, B4Y = 4, B4Z = 2;
+constexpr int N4X = B4X + 3, N4Y = B4Y + 3, N4Z = B4Z + 3;
+constexpr int TILE4 = N4X * N4Y * N4Z;
+// a thread's sums over a cell's queries: ring, c_bar (2), alpha_bar_85
+constexpr int SUMS4 = 35;
+
+struct Sums4 {
+    double ring[4][2][4];
+    double cb[2];
+    double a85;
+};
+
+__device__ __forceinline__ void sums4_zero(Sums4& S) {
 #pragma unroll
-    for (int r = 0; r < PER; ++r) part[o * K + lane + 64 * r] = acc[r];
+    for (int o = 0; o < 4; ++o)
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) S.ring[o][p][e] = 0.0;
+    S.cb[0] = S.cb[1] = S.a85 = 0.0;
 }
 
-constexpr int BWD_CELLS4 = 16;                    // cells per workgroup, 4D
+struct Rec4 {
+    double2 r[5];
+};
 
-template <int D>
-__global__ void __launch_bounds__(256)
-k_bwd_cells(ArbGeom g, const double* __restrict__ A, const double* __restrict__ q, int64_t ldq,
-            const double* __restrict__ gv, const double* __restrict__ gg,
-            const int32_t* __restrict__ offs, const int32_t* __restrict__ perm,
-            const double* __restrict__ part, double* __restrict__ bbar) {
-    constexpr int K = 1 << (2 * D);
-    constexpr int PER = K / 64;
-    constexpr int CB = BWD_CELLS4;
-    static_assert(K == 256, "one thread per entry l of b_bar");
-    __shared__ double abar[CB][K];
-    __shared__ int32_t any;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int64_t c0 = (int64_t)blockIdx.x * CB;
-    if (threadIdx.x == 0) any = 0;
-    __syncthreads();
-    // alpha_bar of the workgroup's cells: wave w forms cells w, w + 4, ...
-    for (int k = w; k < CB; k += 4) {
-        const int64_t c = c0 + k;
-        const bool live = c < g.nc;
-        const int32_t s0 = live ? offs[c] : 0, s1 = live ? offs[c + 1] : 0;
-        double acc[PER];
-        if (s1 - s0 <= BWD_CHUNK) {
-            cell_abar<D, PER>(g, q, ldq, gv, gg, perm, s0, s1, lane, 64, acc);
-        } else {
-            // the queries before the cell's first chunk, then its chunks
-            const int64_t ofirst = ((int64_t)s0 + BWD_CHUNK - 1) / BWD_CHUNK;
-            const int32_t h1 = ofirst * BWD_CHUNK < s1 ? (int32_t)(ofirst * BWD_CHUNK) : s1;
-            cell_abar<D, PER>(g, q, ldq, gv, gg, perm, s0, h1, lane, 64, acc);
-            for (int64_t o = ofirst; o * BWD_CHUNK < s1; ++o) {
+__device__ __forceinline__ Rec4 load_rec4(const double* __restrict__ rec, int64_t s) {
+    Rec4 x;
+    const double2* r2 = reinterpret_cast<const double2*>(rec + s * REC4);
 #pragma unroll
-                for (int r = 0; r < PER; ++r) acc[r] += part[o * K + lane + 64 * r];
+    for (int k = 0; k < 5; ++k) x.r[k] = r2[k];
+    return x;
+}
+
+// Hermite end weight of end m and its derivative: x (c1 + c2 x + x^2) with
+// (c1, c2) = (1, -2) or (0, -1)
+__device__ __forceinline__ void hend(double x, int m, double& h, double& dh) {
+    const double c1 = m ? 0.0 : 1.0, c2 = m ? -1.0 : -2.0;
+    h = x * fma(x, x + c2, c1);
+    dh = fma(x, fma(3.0, x, 2.0 * c2), c1);
+}
+
+// One query's contribution to the sums of thread gq of its cell.
+__device__ __forceinline__ void sums4_row(const Rec4& x, int gq, Sums4& S) {
+    const double u = x.r[0].x, v = x.r[0].y, w = x.r[1].x, t = x.r[1].y;
+    const double gv = x.r[2].x, ku = x.r[2].y, kv = x.r[3].x, kw = x.r[3].y, kt = x.r[4].x;
+    double wt[4], dwt[4];
+    {
+        const double t2 = t * t, t3 = t2 * t;
+#pragma unroll
+        for (int o = 0; o < 4; ++o) {
+            wt[o] = mcol(o, 1.0, t, t2, t3);
+            dwt[o] = mcol(o, 0.0, 1.0, 2.0 * t, 3.0 * t2);
+        }
+    }
+    const int exh = gq & 1, ey = gq >> 1;          // ex = 2 exh + p
+    const double u2 = u * u, v2 = v * v, w2 = w * w;
+    const double pv = ey == 0 ? 1.0 : ey == 1 ? v : ey == 2 ? v2 : v2 * v;
+    const double dv = ey == 0 ? 0.0 : ey == 1 ? 1.0 : ey == 2 ? 2.0 * v : 3.0 * v2;
+    const double pw[4] = {1.0, w, w2, w2 * w}, dw[4] = {0.0, 1.0, 2.0 * w, 3.0 * w2};
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const double pu = exh ? (p ? u2 * u : u2) : (p ? u : 1.0);
+        const double du = exh ? (p ? 3.0 * u2 : 2.0 * u) : (p ? 1.0 : 0.0);
+        const double a = pu * pv;
+        const double base = fma(kv, pu * dv, fma(ku, du * pv, gv * a));
+        const double wa = kw * a, ta = kt * a;
+#pragma unroll
+        for (int ez = 0; ez < 4; ++ez) {
+            const double Q = fma(wa, dw[ez], base * pw[ez]), E = ta * pw[ez];
+#pragma unroll
+            for (int o = 0; o < 4; ++o)
+                S.ring[o][p][ez] = fma(E, dwt[o], fma(Q, wt[o], S.ring[o][p][ez]));
+        }
+    }
+    // c_bar of the corners gq (t end 0) and gq + 8 (t end 1)
+    double hx, dx, hy, dy, hz, dz;
+    hend(u, gq & 1, hx, dx);
+    hend(v, (gq >> 1) & 1, hy, dy);
+    hend(w, gq >> 2, hz, dz);
+    const double hxy = hx * hy, m = hxy * hz;
+    const double Qc = fma(kw, hxy * dz, fma(kv, hx * dy * hz, fma(ku, dx * hy * hz, gv * m)));
+    const double Ec = kt * m;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        double ht, dt;
+        hend(t, e, ht, dt);
+        S.cb[e] = fma(Ec, dt, fma(Qc, ht, S.cb[e]));
+    }
+    // alpha_bar_85: the monomial u v w t
+    const double uv = u * v, q85 = fma(kw, uv, fma(kv, u * w, fma(ku, v * w, gv * (uv * w))));
+    S.a85 = fma(kt, uv * w, fma(q85, t, S.a85));
+}
+
+// The queries at sorted positions [s0, s1), in order.
+__device__ __forceinline__ void sums4_rows(const double* __restrict__ rec, int32_t s0, int32_t s1,
+                                           int gq, Sums4& S) {
+    for (int32_t s = s0; s < s1; ++s) sums4_row(load_rec4(rec, s), gq, S);
+}
+
+// Chunk sums (cells of more than BWD_CHUNK queries): eight threads per
+// chunk, part[o][sum][gq].
+__global__ void __launch_bounds__(256)
+k_bwd_chunk4(ArbGeom g, const double* __restrict__ q, int64_t ldq, const double* __restrict__ rec,
+             const int32_t* __restrict__ offs, const int32_t* __restrict__ perm, int64_t nchunk,
+             double* __restrict__ part) {
+    const int64_t o = (int64_t)blockIdx.x * 32 + (threadIdx.x >> 3);
+    const int gq = threadIdx.x & 7;
+    int32_t s0, s1;
+    if (o >= nchunk || !bwd_chunk<4>(g, q, ldq, offs, perm, o, &s0, &s1)) return;
+    Sums4 S;
+    sums4_zero(S);
+    sums4_rows(rec, s0, s1, gq, S);
+    double* p = part + o * (8 * SUMS4) + gq;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) p[8 * i] = S.ring[i >> 3][(i >> 2) & 1][i & 3];
+    p[8 * 32] = S.cb[0];
+    p[8 * 33] = S.cb[1];
+    p[8 * 34] = S.a85;
+}
+
+__global__ void __launch_bounds__(256)
+k_bwd_block4(ArbGeom g, const double* __restrict__ rec, const int32_t* __restrict__ offs,
+             int64_t nbx, int64_t nby, const double* __restrict__ part,
+             double* __restrict__ tiles) {
+    // [z][cy][cx][ex + 4 ey] and [z][y][cx][ex]; a plane of t2 and a row of t1
+    // padded so that the threads of the y and x passes spread over the banks
+    constexpr int P2 = B4Y * B4X * 16 + 12, P1 = B4X * 4 + 2;
+    __shared__ __align__(16) double t2[N4Z * P2];
+    __shared__ __align__(16) double t1[N4Z * N4Y * P1];
+    __shared__ __align__(16) double gb[B4X * B4Y * B4Z][16];    // G_bar per cell
+    const int64_t blk = blockIdx.x;
+    const int64_t bx = blk % nbx, by = (blk / nbx) % nby, bz = blk / (nbx * nby);
+    const int cl = threadIdx.x >> 3, gq = threadIdx.x & 7;
+    const int cx = cl & 3, cy = (cl >> 2) & 3, cz = cl >> 4;
+    const int64_t x = bx * B4X + cx, y = by * B4Y + cy, z = bz * B4Z + cz;
+    const bool in = x < g.npos[0] && y < g.npos[1] && z < g.npos[2];
+    const int64_t c0 = x + g.npos[0] * (y + g.npos[1] * z);
+    const int64_t layer = g.npos[0] * g.npos[1] * g.npos[2];
+    const int32_t nct = (int32_t)g.npos[3], nt = (int32_t)g.n[3];
+    double* out = tiles + blk * nt * TILE4;
+    Sums4 S;
+    sums4_zero(S);
+    int idle = 4;                                    // layers since the last query
+    // the bounds of the next layer's cell are loaded before this layer's sums
+    int32_t n0 = 0, n1 = 0;
+    auto fetch = [&](int32_t ct) {
+        n0 = n1 = 0;
+        if (in && ct < nct) {
+            const int64_t c = c0 + layer * ct;
+            n0 = offs[c];
+            n1 = offs[c + 1];
+        }
+    };
+    fetch(0);
+    for (int32_t ct = 0; ct < nt; ++ct) {
+        const int32_t s0 = n0, s1 = n1;
+        fetch(ct + 1);
+        idle = __syncthreads_or(s1 > s0) ? 0 : idle + 1;
+        if (idle > 3) {                              // nothing in reach of this plane
+            for (int t = threadIdx.x; t < TILE4; t += 256) out[(int64_t)ct * TILE4 + t] = 0.0;
+            continue;
+        }
+        if (idle == 0) {
+            S.cb[0] = S.cb[1] = S.a85 = 0.0;
+            if (s1 - s0 <= BWD_CHUNK) {
+                sums4_rows(rec, s0, s1, gq, S);
+            } else {
+                // the queries before the cell's first chunk, then its chunks
+                const int64_t ofirst = ((int64_t)s0 + BWD_CHUNK - 1) / BWD_CHUNK;
+                const int32_t h1 = ofirst * BWD_CHUNK < s1 ? (int32_t)(ofirst * BWD_CHUNK) : s1;
+                sums4_rows(rec, s0, h1, gq, S);
+                for (int64_t o = ofirst; o * BWD_CHUNK < s1; ++o) {
+                    const double* p = part + o * (8 * SUMS4) + gq;
+#pragma unroll
+                    for (int i = 0; i < 32; ++i) S.ring[i >> 3][(i >> 2) & 1][i & 3] += p[8 * i];
+                    S.cb[0] += p[8 * 32];
+                    S.cb[1] += p[8 * 33];
+                    S.a85 += p[8 * 34];
+                }
+            }
+            // alpha_85 = 0: its part of the sums (M[1][ot] along t; P's column 0)
+            if (gq == 2) {
+                S.ring[0][1][1] += 0.5 * S.a85;
+                S.ring[2][1][1] -= 0.5 * S.a85;
+            }
+            if (gq == 0) S.cb[0] -= S.a85;
+            // G_bar(j) = c_bar_{j+1} - c_bar_j, corners j = gq and gq + 8
+            const int lane = threadIdx.x & 63, nl = (lane & ~7) | ((gq + 1) & 7);
+            const double n0 = __shfl(S.cb[0], nl), n1 = __shfl(S.cb[1], nl);
+            gb[cl][gq] = (gq == 7 ? n1 : n0) - S.cb[0];
+            gb[cl][gq + 8] = (gq == 7 ? 0.0 : n1) - S.cb[1];
+            __syncthreads();
+            // ring += X (x) X (x) X G_bar in (ex, ey, ez), the differences along t
+            const int exh = gq & 1, ey = gq >> 1;
+            if (ey) {
+                const double ya = ey == 1 ? 1.0 : 0.0, yb = (double)ey;
+#pragma unroll
+                for (int mt = 0; mt < 2; ++mt) {
+                    double r[2][2];                  // [mx][mz], summed over my
+#pragma unroll
+                    for (int mz = 0; mz < 2; ++mz)
+#pragma unroll
+                        for (int mx = 0; mx < 2; ++mx)
+                            r[mx][mz] = fma(yb, gb[cl][mx + 2 + 4 * mz + 8 * mt],
+                                            ya * gb[cl][mx + 4 * mz + 8 * mt]);
+#pragma unroll
+                    for (int p = 0; p < 2; ++p) {
+                        const int ex = 2 * exh + p;
+                        if (ex == 0) continue;
+                        const double xa = ex == 1 ? 1.0 : 0.0, xb = (double)ex;
+                        const double z0 = fma(xb, r[1][0], xa * r[0][0]);
+                        const double z1 = fma(xb, r[1][1], xa * r[0][1]);
+                        const double e[4] = {0.0, z0 + z1, 2.0 * z1, 3.0 * z1};
+#pragma unroll
+                        for (int ez = 1; ez < 4; ++ez) {
+                            S.ring[mt][p][ez] -= 0.5 * e[ez];
+                            S.ring[mt + 2][p][ez] += 0.5 * e[ez];
+                        }
+                    }
+                }
             }
         }
+        // plane ct.  z: t2[z][cy][cx][exy] = sum over cz + oz = z of
+        // sum_ez M[ez][oz] ring[0][exy][ez], the lower cell layer first
 #pragma unroll
-        for (int r = 0; r < PER; ++r) abar[k][lane + 64 * r] = acc[r];
-        if (s0 != s1 && lane == 0) any = 1;
-    }
-    __syncthreads();
-    // b_bar[l][c] = sum_j A[j][l] alpha_bar[c][j], j ascending from 0, for
-    // the CB cells at once: thread l reads each A[j][l] once (a row of A is
-    // one coalesced read) and alpha_bar[c][j] is an LDS broadcast.  A cell
-    // without queries gets 0.
-    const int l = threadIdx.x;
-    double b[CB];
+        for (int ph = 0; ph < B4Z; ++ph) {
+            if (cz == ph) {
 #pragma unroll
-    for (int k = 0; k < CB; ++k) b[k] = 0.0;
-    if (any) {
-        for (int j = 0; j < K; ++j) {
-            const double a = A[(int64_t)j * K + l];
-#pragma unroll
-            for (int k = 0; k < CB; ++k) b[k] += a * abar[k][j];
+                for (int oz = 0; oz < 4; ++oz) {
+                    double2* o = reinterpret_cast<double2*>(t2 + (ph + oz) * P2 + (4 * cy + cx) * 16 + 2 * gq);
+                    double2 b = make_double2(
+                        mcol(oz, S.ring[0][0][0], S.ring[0][0][1], S.ring[0][0][2], S.ring[0][0][3]),
+                        mcol(oz, S.ring[0][1][0], S.ring[0][1][1], S.ring[0][1][2], S.ring[0][1][3]));
+                    if (ph > 0 && oz < 3) {
+                        b.x += o->x;
+                        b.y += o->y;
+                    }
+                    *o = b;
+                }
+            }
+            __syncthreads();
         }
-    }
+        // y: t1[z][y][cx][ex] = sum_{cy + oy = y} sum_ey M[ey][oy] t2[z][cy][cx][ex + 4 ey],
+        // a thread per (z, cx, ex): its 16 values read once, 7 sums
+        if (threadIdx.x < N4Z * B4X * 4) {
+            const int ex = threadIdx.x & 3, tx = (threadIdx.x >> 2) & 3, zz = threadIdx.x >> 4;
+            double sum[N4Y];
 #pragma unroll
-    for (int k = 0; k < CB; ++k) {
-        const int64_t c = c0 + k;
-        if (c < g.nc) {
-            const int32_t s0 = offs[c], s1 = offs[c + 1];
-            bbar[(int64_t)l * g.nc + c] = s0 != s1 ? b[k] : 0.0;
+            for (int i = 0; i < N4Y; ++i) sum[i] = 0.0;
+#pragma unroll
+            for (int ty = 0; ty < B4Y; ++ty) {
+                const double* a = t2 + zz * P2 + (4 * ty + tx) * 16 + ex;
+                const double a0 = a[0], a1 = a[4], a2 = a[8], a3 = a[12];
+#pragma unroll
+                for (int oy = 0; oy < 4; ++oy) sum[ty + oy] += mcol(oy, a0, a1, a2, a3);
+            }
+#pragma unroll
+            for (int i = 0; i < N4Y; ++i) t1[(zz * N4Y + i) * P1 + 4 * tx + ex] = sum[i];
         }
+        __syncthreads();
+        // x: the plane's nodes, sum_{cx + ox = x} sum_ex M[ex][ox] t1[z][y][cx][ex],
+        // a thread per (z, y) row
+        if (threadIdx.x < N4Z * N4Y) {
+            const double* a = t1 + threadIdx.x * P1;
+            double sum[N4X];
+#pragma unroll
+            for (int i = 0; i < N4X; ++i) sum[i] = 0.0;
+#pragma unroll
+            for (int tx = 0; tx < B4X; ++tx)
+#pragma unroll
+                for (int ox = 0; ox < 4; ++ox)
+                    sum[tx + ox] += mcol(ox, a[4 * tx], a[4 * tx + 1], a[4 * tx + 2], a[4 * tx + 3]);
+            double* o = out + (int64_t)ct * TILE4 + threadIdx.x * N4X;
+#pragma unroll
+            for (int i = 0; i < N4X; ++i) o[i] = sum[i];
+        }
+        // the ring moves on by one plane
+#pragma unroll
+        for (int o = 0; o < 4; ++o)
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) S.ring[o][p][e] = o < 3 ? S.ring[o + 1][p][e] : 0.0;
     }
 }
 
-// Node adjoint: gather b_bar from the cells whose neighbourhood holds the node.
-template <int D>
+// Node gradient: the sum, over the blocks whose tile holds the node (at most
+// two in x and y, three in z), of the tile entries, blocks in ascending z, y,
+// x order.
 __global__ void __launch_bounds__(256)
-k_bwd_nodes(ArbGeom g, const double* __restrict__ bbar, double* __restrict__ dval) {
-    constexpr int K = 1 << (2 * D);
+k_bwd_nodes4(ArbGeom g, const double* __restrict__ tiles, int64_t nbx, int64_t nby, int64_t nbz,
+             double* __restrict__ dval) {
     const int64_t nidx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (nidx >= g.nnodes) return;
-    int64_t x[D];
-    int64_t rem = nidx;
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-        x[a] = rem % g.n[a];
-        rem /= g.n[a];
-    }
+    const int64_t i = nidx % g.n[0], j = (nidx / g.n[0]) % g.n[1];
+    const int64_t r = nidx / (g.n[0] * g.n[1]), k = r % g.n[2], t = r / g.n[2];
+    // the first block of edge b whose tile (b + 3 nodes) reaches node v
+    auto lo = [](int64_t v, int b) { const int64_t w = v - (b + 2); return w <= 0 ? (int64_t)0 : (w + b - 1) / b; };
+    const int64_t x0 = lo(i, B4X), x1 = min(i / B4X, nbx - 1);
+    const int64_t y0 = lo(j, B4Y), y1 = min(j / B4Y, nby - 1);
+    const int64_t z0 = lo(k, B4Z), z1 = min(k / B4Z, nbz - 1);
     double sum = 0.0;
-    for (int l = 0; l < K; ++l) {          // neighbour slot l: offsets o_a = (l >> 2a) & 3
-        int64_t cell = 0, mul = 1;
-        bool ok = true;
-#pragma unroll
-        for (int a = 0; a < D; ++a) {
-            const int64_t ca = x[a] - ((l >> (2 * a)) & 3);
-            ok &= (ca >= 0) && (ca < g.npos[a]);
-            cell += ca * mul;
-            mul *= g.npos[a];
-        }
-        if (ok) sum += bbar[(int64_t)l * g.nc + cell];
-    }
+    for (int64_t bz = z0; bz <= z1; ++bz)
+        for (int64_t by = y0; by <= y1; ++by)
+            for (int64_t bx = x0; bx <= x1; ++bx) {
+                const int64_t blk = bx + nbx * (by + nby * bz);
+                const int64_t e = (i - B4X * bx) + N4X * ((j - B4Y * by) + N4Y * (k - B4Z * bz));
+                sum += tiles[(blk * g.n[3] + t) * TILE4 + e];
+            }
     dval[nidx] = sum;
 }
 
@@ -638,52 +817,62 @@ void arb_bwd_blocks3(const ArbGeom& g, int64_t* nb3) {
     for (int a = 0; a < 3; ++a) nb3[a] = (g.npos[a] + BB - 1) / BB;
 }
 
+int64_t arb_bwd_rec_elems(const ArbGeom& g) { return g.ndim == 3 ? 8 : REC4; }
+
+void arb_bwd_blocks4(const ArbGeom& g, int64_t* nb4) {
+    nb4[0] = (g.npos[0] + B4X - 1) / B4X;
+    nb4[1] = (g.npos[1] + B4Y - 1) / B4Y;
+    nb4[2] = (g.npos[2] + B4Z - 1) / B4Z;
+}
+
 int64_t arb_bwd_scratch(const ArbGeom& g) {
+    int64_t nb[3];
     if (g.ndim == 3) {
-        int64_t nb3[3];
-        arb_bwd_blocks3(g, nb3);
-        return nb3[0] * nb3[1] * nb3[2] * BTILE;
+        arb_bwd_blocks3(g, nb);
+        return nb[0] * nb[1] * nb[2] * BTILE;
     }
-    return g.nc * 256;
+    arb_bwd_blocks4(g, nb);
+    return nb[0] * nb[1] * nb[2] * g.n[3] * TILE4;
 }
 
 int64_t arb_bwd_part_elems(const ArbGeom& g, int64_t n) {
     const int64_t nchunk = (n + BWD_CHUNK - 1) / BWD_CHUNK;
-    return (nchunk ? nchunk : 1) * (g.ndim == 3 ? 64 : 256);
+    return (nchunk ? nchunk : 1) * (g.ndim == 3 ? 64 : 8 * SUMS4);
 }
 
-hipError_t arb_launch_bwd_cells(const ArbGeom& g, const double* A, const double* q, int64_t ldq,
-                                const double* gv, const double* gg, const double* rec,
+hipError_t arb_launch_bwd_cells(const ArbGeom& g, const double* q, int64_t ldq, const double* rec,
                                 int32_t rec_grouped, const int32_t* offs, const int32_t* perm,
                                 int64_t n, double* part, double* bbar, hipStream_t s) {
     const int32_t* rperm = rec_grouped ? nullptr : perm;
     const int64_t nchunk = (n + BWD_CHUNK - 1) / BWD_CHUNK;
+    int64_t nb[3];
     if (g.ndim == 3) {
         if (nchunk > 0)
             hipLaunchKernelGGL(k_bwd_chunk3, dim3(grid1(nchunk, 64)), dim3(256), 0, s, g, q, ldq,
                                rec, offs, perm, rperm, nchunk, part);
-        int64_t nb3[3];
-        arb_bwd_blocks3(g, nb3);
-        hipLaunchKernelGGL(k_bwd_block3, dim3((unsigned)(nb3[0] * nb3[1] * nb3[2])), dim3(256), 0,
-                           s, g, rec, offs, rperm, nb3[0], nb3[1], (const double*)part, bbar);
+        arb_bwd_blocks3(g, nb);
+        hipLaunchKernelGGL(k_bwd_block3, dim3((unsigned)(nb[0] * nb[1] * nb[2])), dim3(256), 0,
+                           s, g, rec, offs, rperm, nb[0], nb[1], (const double*)part, bbar);
     } else {
         if (nchunk > 0)
-            hipLaunchKernelGGL(k_bwd_chunk<4>, dim3(grid1(nchunk, 4)), dim3(256), 0, s, g, q, ldq,
-                               gv, gg, offs, perm, nchunk, part);
-        hipLaunchKernelGGL(k_bwd_cells<4>, dim3(grid1(g.nc, BWD_CELLS4)), dim3(256), 0, s, g, A,
-                           q, ldq, gv, gg, offs, perm, (const double*)part, bbar);
+            hipLaunchKernelGGL(k_bwd_chunk4, dim3(grid1(nchunk, 32)), dim3(256), 0, s, g, q, ldq,
+                               rec, offs, perm, nchunk, part);
+        arb_bwd_blocks4(g, nb);
+        hipLaunchKernelGGL(k_bwd_block4, dim3((unsigned)(nb[0] * nb[1] * nb[2])), dim3(256), 0,
+                           s, g, rec, offs, nb[0], nb[1], (const double*)part, bbar);
     }
     return hipGetLastError();
 }
 
 hipError_t arb_launch_bwd_nodes(const ArbGeom& g, const double* bbar, double* dval, hipStream_t s) {
     dim3 grid(grid1(g.nnodes, 256)), block(256);
+    int64_t nb[3];
     if (g.ndim == 3) {
-        int64_t nb3[3];
-        arb_bwd_blocks3(g, nb3);
-        hipLaunchKernelGGL(k_bwd_nodes3, grid, block, 0, s, g, bbar, nb3[0], nb3[1], nb3[2], dval);
+        arb_bwd_blocks3(g, nb);
+        hipLaunchKernelGGL(k_bwd_nodes3, grid, block, 0, s, g, bbar, nb[0], nb[1], nb[2], dval);
     } else {
-        hipLaunchKernelGGL(k_bwd_nodes<4>, grid, block, 0, s, g, bbar, dval);
+        arb_bwd_blocks4(g, nb);
+        hipLaunchKernelGGL(k_bwd_nodes4, grid, block, 0, s, g, bbar, nb[0], nb[1], nb[2], dval);
     }
     return hipGetLastError();
 }
