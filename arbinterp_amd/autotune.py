@@ -7,7 +7,7 @@ on the caller's own positions (GPU, HIP events on the current stream):
   * the cell-bucketed kernel staging coefficients from the table
     (ARB_Q_TABLE) and the default bucketed kernel, for every block of cells
     (cells per axis) on a ladder whose LDS footprint fits, with 64/128/256
-    threads per workgroup.
+    threads per workgroup; and the bucketed path as the library chooses it.
 
 Outputs that must not depend on the launch shape are compared bit for bit:
 every table-staged candidate against the first one, and the default
@@ -116,7 +116,7 @@ def tune_query(interp, q, reps=3, max_candidates=None, verify=True, use_cache=Tr
         return dict(best, cached=True)
     out = interp.query_device(q, flags=N.ARB_Q_DIRECT)
     ref = tuple(t.clone() if t is not None else None for t in out)
-    cands = [("direct", None, 0)]
+    cands = [("direct", None, 0), ("sorted", None, 0)]
     for b in block_ladder(interp):
         for th in (64, 128, 256):
             cands.append(("table", b, th))

@@ -185,8 +185,8 @@ struct arb_field {
     int64_t table_bytes = 0;
     void* sent = nullptr;       // [ninterp][K] the sentinel row, for paths without the table
     int32_t* flag = nullptr;    // device status word
-    // bucketed query path: block geometry of the table kernels (B) and of the
-    // fused kernel (BF, without the larger blocks that only save a sort pass)
+    // bucketed query path: block geometry of the table and node-tile kernels
+    // (B) and of the on-the-fly kernels (BF)
     ArbBuckets B{};
     ArbBuckets BF{};
     int32_t user_block[ARB_MAXD] = {0, 0, 0, 0};
@@ -239,17 +239,20 @@ struct arb_field {
 
 // Choose the cell block of one bucket: the largest of a fixed ladder whose
 // coefficients (padded by 16 bytes per cell) fit in 48 KiB of LDS, unless the
-// caller set one.  With `upgrade`, when that leaves 2^16 buckets or more (a
-// third 8-bit radix pass), a larger block within 80 KiB that brings the
-// count below 2^16 is taken instead: on the 128^3 FP64 field this trades
-// 0.06 ms of evaluation (fewer workgroups per CU) for a 0.08 ms sort pass.
+// caller set one.  For the table kernels (`table`), when that leaves 2^16
+// buckets or more (a third 8-bit radix pass), a larger block within 80 KiB
+// that brings the count below 2^16 is taken instead: on the 128^3 FP64 field
+// this trades 0.06 ms of evaluation (fewer workgroups per CU) for a 0.08 ms
+// sort pass.  The 3D on-the-fly kernel stores no coefficients: its largest
+// block, 4 x 4 x 4, forms the fewest passes per cell and has rows for every
+// wave (128^3 FP64 'both', 10^7 rows: 0.94 ms; 4 x 4 x 2 cells: 1.7 ms).
 static int64_t bucket_count(const arb_field* f, const int* dims) {
     int64_t nb = 1;
     for (int a = 0; a < f->g.ndim; ++a) nb *= (f->g.npos[a] + dims[a] - 1) / dims[a];
     return nb;
 }
 
-static void choose_buckets(arb_field* f, ArbBuckets& B, bool upgrade) {
+static void choose_buckets(arb_field* f, ArbBuckets& B, bool table) {
     const int d = f->g.ndim;
     const int K = 1 << (2 * d);
     const int esz = f->precision == ARB_PREC_FP64 ? 8 : 4;
@@ -281,9 +284,9 @@ static void choose_buckets(arb_field* f, ArbBuckets& B, bool upgrade) {
         };
         int pick = -1;
         for (int i = 0; i < nl && pick < 0; ++i)
-            if (cells(i) <= max_cells) pick = i;
+            if (cells(i) <= max_cells || (d == 3 && !table)) pick = i;
         if (pick < 0) pick = nl - 1;
-        if (upgrade && count(pick) >= ((int64_t)1 << 16))
+        if (table && count(pick) >= ((int64_t)1 << 16))
             for (int i = pick - 1; i >= 0; --i)
                 if (cells(i) <= big_cells && count(i) < ((int64_t)1 << 16)) {
                     pick = i;
@@ -533,6 +536,7 @@ int arb_field_create(const double* rows_dev, int64_t nrows, int32_t ncols, int64
         g.npos[a] = g.n[a] - 3;
         g.nc *= g.npos[a];
         g.h[a] = std::fabs(axes[a][0] - axes[a][1]);
+        g.rh[a] = arb_recip(g.h[a]);
         g.lo[a] = axes[a][1];
         g.hi[a] = axes[a][g.n[a] - 2];
         f->edge_lo[a] = axes[a][0];
@@ -819,14 +823,25 @@ static int query_impl(arb_field* f, double* q_dev, int64_t n, int64_t ldq, void*
         sorted = n >= 65536 && (node_path(f, flags) ? 4 * n : 2 * n) >= f->g.nc;
     if (n > INT32_MAX - 1) sorted = false;
     if (sorted && f->B.nbt == 0) choose_buckets(f, f->B, true);
-    // 3D, bucketed, on request: coefficients formed in the query kernel from
-    // node values, no table (ignored once a table has been loaded, or when
-    // the block does not fit the kernel's LDS)
+    // 3D, bucketed: coefficients formed in the query kernel from node values,
+    // no table, with the table's bits (not once a table has been loaded).  On
+    // request, and by itself for FP64 fields of three or four interpolants
+    // whose table is larger than the Infinity Cache: measured against the
+    // table kernel (evaluation, ms) 0.94 / 1.33 for 'both' on 128^3 nodes and
+    // 10^7 rows (3.8 GB of table), 0.265 / 0.38 on 112 x 96 x 88 and 10^6 rows,
+    // 0.078 / 0.111 for 'vector' on 97 x 61 x 45 and 10^6 rows (335 MB), but
+    // 0.044 / 0.042 for a table of 107 MB, which stays cached; one interpolant
+    // gains nothing either (0.29 / 0.25 on 128^3 and 2 10^6 rows).  A block
+    // chosen by the caller is the table kernel's.
+    constexpr int64_t kInfinityCache = (int64_t)256 << 20;
+    const bool by_size = f->precision == ARB_PREC_FP64 && f->ninterp >= 3 &&
+                         f->table_bytes > kInfinityCache && f->user_block[0] == 0 && !noalloc &&
+                         !(flags & ARB_Q_TABLE);
     bool fused = false;
-    if ((flags & ARB_Q_FUSED) && sorted && f->g.ndim == 3 && !f->table_loaded &&
+    if (((flags & ARB_Q_FUSED) || by_size) && sorted && f->g.ndim == 3 && !f->table_loaded &&
         !(flags & (ARB_Q_SORTED_GLOBAL | ARB_Q_GROUP_ATOMIC))) {
         if (f->BF.nbt == 0) choose_buckets(f, f->BF, false);
-        fused = arb_fused_lds(f->g, f->BF, f->ninterp, f->eval_threads) > 0;
+        fused = arb_fused_ok(f->g, f->BF, f->ninterp);
     }
     // node tiles (mixed 3D): the direct path, and the bucketed path unless
     // another grouping or the fused kernel is asked for; no table
@@ -849,7 +864,7 @@ static int query_impl(arb_field* f, double* q_dev, int64_t n, int64_t ldq, void*
         sorted = true;
         if (f->BF.nbt == 0) choose_buckets(f, f->BF, false);
         if (f->g.ndim == 3)
-            fused = arb_fused_lds(f->g, f->BF, f->ninterp, f->eval_threads) > 0;
+            fused = arb_fused_ok(f->g, f->BF, f->ninterp);
         else
             fused4 = arb_fused4_lds(f->g, f->BF) > 0;
         if (!fused && !fused4)
@@ -1048,9 +1063,8 @@ static int query_impl(arb_field* f, double* q_dev, int64_t n, int64_t ldq, void*
             HIPCHK(arb_launch_eval_nodes(f->g, BB, f->ninterp, out64, f->tiles, w.qrec, qstride,
                                          n, o, offs, perm, hot, f->eval_threads, s));
         else if (fused)
-            HIPCHK(arb_launch_eval_fused(f->g, BB, f->precision, out64, f->vals, f->ninterp,
-                                         f->has_comps, f->has_norm, q_dev, n, ldq, o, offs,
-                                         perm, hot, f->eval_threads, s));
+            HIPCHK(arb_launch_eval_fused(f->g, BB, f->precision, out64, f->vals, f->ninterp, q_dev,
+                                         n, ldq, o, offs, perm, hot, s));
         else if (fused4)
             HIPCHK(arb_launch_eval_fused4(f->g, BB, f->precision, out64, f->vals, f->ninterp,
                                           f->has_comps, f->has_norm, q_dev, n, ldq, o, offs,

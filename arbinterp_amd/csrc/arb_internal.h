@@ -14,6 +14,7 @@ struct ArbGeom {
     double lo[ARB_MAXD];      // IntMin per axis
     double hi[ARB_MAXD];      // IntMax per axis
     double h[ARB_MAXD];       // spacing |node0 - node1|
+    double rh[ARB_MAXD];      // 1 / h, or 0 where arb_div_h must divide (arb_recip)
     int64_t n[ARB_MAXD];      // nodes per axis
     int64_t npos[ARB_MAXD];   // cells per axis = n - 3
     int64_t nstride[ARB_MAXD];// node strides (x fastest)
@@ -85,6 +86,26 @@ __device__ __forceinline__ void arb_reduce_axis(double x, const ArbGeom& g, int 
         *fl = floor(*iu);
         *loc = *iu - *fl;
     }
+}
+
+// a / h[axis], the IEEE quotient, from rh = 1 / h correctly rounded (P.
+// Markstein, "Computation of elementary functions on the IBM RISC System/6000
+// processor", IBM J. Res. Dev. 34, 1990): a rh is within 1.5 units in the last
+// place, the residual a - q h is exact, one correction gives a quotient within
+// one unit in the last place and the second the correctly rounded one, as long
+// as nothing under- or overflows.  Five FP64 operations, where the general
+// division takes about fourteen issue slots (it scales, starts from a
+// quarter-rate reciprocal and fixes up).  rh = 0 stands for a spacing so small
+// or large that a residual could leave the range: such grids divide.
+__host__ __device__ inline double arb_recip(double h) {
+    return h > 0x1p-300 && h < 0x1p300 ? 1.0 / h : 0.0;
+}
+__device__ __forceinline__ double arb_div_h(double a, const ArbGeom& g, int axis) {
+    const double h = g.h[axis], rh = g.rh[axis];
+    if (rh == 0.0) return a / h;
+    double q = a * rh;
+    q = fma(fma(-q, h, a), rh, q);
+    return fma(fma(-q, h, a), rh, q);
 }
 
 template <int D>
@@ -314,12 +335,13 @@ hipError_t arb_launch_group_sort(const uint32_t* keys, uint32_t* ent, int32_t* p
                                  int64_t nbt, int32_t* kcnt, hipStream_t s);
 hipError_t arb_launch_scatter(const int32_t* bkt, const int32_t* rank, const int32_t* offs,
                               int32_t* perm, int64_t n, hipStream_t s);
-size_t arb_fused_lds(const ArbGeom& g, const ArbBuckets& B, int32_t ninterp, int32_t threads);
+// 3D bucketed query without the table; ARB_EVAL_CHUNK rows at most per
+// workgroup (its grid: buckets, then chunks).
+bool arb_fused_ok(const ArbGeom& g, const ArbBuckets& B, int32_t ninterp);
 hipError_t arb_launch_eval_fused(const ArbGeom& g, const ArbBuckets& B, int32_t prec,
                                  int32_t out_f64, const double* vals, int32_t ninterp,
-                                 int32_t has_comps, int32_t has_norm, const double* q, int64_t n,
-                                 int64_t ldq, const ArbOut& o, const int32_t* offs,
-                                 const int32_t* perm, const int32_t* hot, int32_t block_threads,
+                                 const double* q, int64_t n, int64_t ldq, const ArbOut& o,
+                                 const int32_t* offs, const int32_t* perm, const int32_t* hot,
                                  hipStream_t s);
 // 4D bucketed query without the table (coefficients formed per bucket with
 // the 4D table build's arithmetic); arb_fused4_lds is 0 where it does not

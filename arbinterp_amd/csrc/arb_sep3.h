@@ -45,10 +45,11 @@ __device__ void cell_bad3(const double* nodes, unsigned char* bad) {
     for (int c = threadIdx.x; c < BX * BY * BZ; c += blockDim.x) {
         const int cx = c % BX, cy = (c / BX) % BY, cz = c / (BX * BY);
         bool b = false;
-        for (int z = 0; z < 4; ++z)
-            for (int y = 0; y < 4; ++y)
-                for (int x = 0; x < 4; ++x)
-                    b |= !isfinite(nodes[((cz + z) * NY + cy + y) * NX + cx + x]);
+        // not unrolled: this rare path must not set the callers' registers
+#pragma unroll 1
+        for (int zy = 0; zy < 16; ++zy)
+            for (int x = 0; x < 4; ++x)
+                b |= !isfinite(nodes[((cz + (zy >> 2)) * NY + cy + (zy & 3)) * NX + cx + x]);
         bad[c] = b ? 1 : 0;
     }
 }

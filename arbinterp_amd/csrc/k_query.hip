@@ -283,6 +283,21 @@ __device__ __forceinline__ int64_t bucket_of(int64_t flat, const int64_t* ia, co
     return bidx;
 }
 
+// First cell of bucket b.  Buckets are counted in 32 bits (the launchers put
+// one workgroup on each): the divisions are 32-bit ones, where 64-bit ones
+// take about 140 scalar instructions each, a microsecond before a workgroup
+// can start its loads.
+template <int D>
+__device__ __forceinline__ void bucket_origin(int64_t b, const ArbBuckets& B, int64_t* c0) {
+    uint32_t rem = (uint32_t)b;
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+        const uint32_t nb = (uint32_t)B.nb[a], up = a + 1 < D ? rem / nb : 0;
+        c0[a] = (int64_t)(a + 1 < D ? rem - up * nb : rem) << B.bsh[a];
+        rem = up;
+    }
+}
+
 // Cell-local coordinates of the node-tile paths, as every one of them (and
 // the per-row records of the bucketed path) carries them: the FP32 value
 // per axis, which the Hermite weights use, plus an 8-bit correction per
@@ -664,18 +679,16 @@ struct StageBase {
 template <int D>
 __device__ __forceinline__ void stage_base(int64_t b, const ArbGeom& g, const ArbBuckets& B,
                                            StageBase<D>& sb) {
-    int64_t rem = b;
+    int64_t c0[D];
+    bucket_origin<D>(b, B, c0);
     uint64_t cell = 0, st = 1;
     bool edge = false;
 #pragma unroll
     for (int a = 0; a < D; ++a) {
-        const int64_t bi = rem % B.nb[a];
-        rem /= B.nb[a];
-        const int64_t c0 = bi << B.bsh[a];
-        const int64_t left = g.npos[a] - c0;
+        const int64_t left = g.npos[a] - c0[a];
         sb.ext[a] = (int32_t)(left < B.b[a] ? left : B.b[a]);
         edge |= sb.ext[a] < B.b[a];
-        cell += (uint64_t)c0 * st;
+        cell += (uint64_t)c0[a] * st;
         st *= (uint64_t)g.npos[a];
     }
     sb.edge = edge;
@@ -826,108 +839,333 @@ k_eval_bucket(ArbGeom g, ArbBuckets B, const TC* __restrict__ table, int32_t has
     }
 }
 
-// 3D without the coefficient table: one workgroup per bucket forms its
-// cells' coefficients from node values (per interpolant: node tile, cells + 3
-// per axis, into LDS, then the separable passes of arb_sep3.h, the routine
-// the table build uses, so the results are bitwise those of the table),
-// writes them into the same LDS block layout the staged kernel uses, and
-// evaluates the bucket's queries.  The node tiles of all interpolants are
-// loaded into registers first (FUSED_REGS per thread, all loads in flight at
-// once), so the passes never wait on global memory.  Dynamic LDS: ncell *
-// cellstride * 16 bytes of coefficients, then one node tile and the pass
-// buffers (doubles).
-constexpr int FUSED_REGS = 8;
+// 3D without the coefficient table: one workgroup per bucket evaluates its
+// rows from node values, in the order of operations of the table build
+// (arb_sep3.h's passes: the cub4 chains along x, y and z) and of the table
+// kernels (arb_val3, arb_valgrad3), so the results are bitwise those of the
+// table.  Per interpolant: the node tile (cells + 3 per axis) goes to LDS, the x
+// and y passes give the 16 (ex, ey) values of every (cell column, node plane)
+// in LDS, and a lane forms the z pass in registers, four coefficients of one
+// (ex, ey) at a time, straight into Horner's rule.
+//
+// So the coefficients themselves are nowhere stored (64 doubles written and
+// read per cell and interpolant otherwise).  A lane takes two rows of one
+// cell, the z pass and its LDS reads shared: the rows are put in cell order
+// first, each cell from an even position (a counting sort in LDS), so item i
+// is the sorted positions 2i and 2i + 1, the second empty for the last row of
+// a cell with an odd number.  Neighbouring lanes read the same or the next
+// cells: LDS broadcasts and different banks.
+//
+// 128^3 FP64 'both', 10^7 rows: 0.94 ms, against 1.33 ms for the staged table
+// kernel (4 GB of coefficients through HBM; here 0.35 GB of nodes); 112 x 96 x
+// 88, 10^6 rows: 0.265 against 0.38 ms.  VALU issue (0.45 ms of the first) and
+// the chain row index -> position -> sort ahead of the passes bound it, at four
+// waves per SIMD (at three: 0.30 ms for the second).  The same kernel with
+// the coefficients of one interpolant at a time in LDS took 1.27 ms (LDS
+// active 0.59 ms of it), of all four 1.5 ms.
+constexpr int FUSED_ROWS = ARB_EVAL_CHUNK / arbs3::SEP_THREADS;
 
-template <typename T, typename TO, int BX, int BY, int BZ>
-__global__ void __launch_bounds__(256)
-k_eval_fused3(ArbGeom g, ArbBuckets B, const double* __restrict__ vals, int32_t ninterp,
-              int32_t has_comps, int32_t has_norm, const double* __restrict__ q, int64_t n,
-              int64_t ldq, ArbOut o, const int32_t* __restrict__ offs,
-              const int32_t* __restrict__ perm, const int32_t* __restrict__ hot) {
-    extern __shared__ uint4 smem[];
+// The reduction of arb_reduce_axes for a row of the BX x BY x BZ cells at c0
+// (in 32 bits); false for any other row (loc and lc are then not valid).
+template <int BX, int BY, int BZ>
+__device__ __forceinline__ bool local_cell(const double* x, const ArbGeom& g, const int64_t* c0,
+                                           double* loc, int* lc) {
+    constexpr int E[3] = {BX, BY, BZ};
+    bool in = true;
+    int l[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        in &= x[a] >= g.lo[a] && x[a] <= g.hi[a];
+        const double iu = arb_div_h(x[a] - g.lo[a], g, a), fl = floor(iu);
+        loc[a] = iu - fl;
+        const double d = fl - (double)c0[a];
+        in &= d >= 0.0 && d < (double)E[a] && fl < (double)g.npos[a];
+        l[a] = in ? (int)d : 0;
+    }
+    *lc = l[0] + BX * (l[1] + BY * l[2]);
+    return in;
+}
+
+// Streaming Horner along v, from the highest power: h4 and h4d of arb_internal.h
+// (the same operations in the same order), with the rows p_j handed over one
+// at a time, j = 3, 2, 1, 0.
+template <typename T>
+__device__ __forceinline__ void stream_h4(int j, T p, T v, T& b) { b = j == 3 ? p : fma(b, v, p); }
+template <typename T>
+__device__ __forceinline__ void stream_h4d(int j, T p, T v, T& b, T& d) {
+    if (j == 3) {
+        b = p;
+    } else if (j == 2) {
+        const T nb = fma(b, v, p);
+        d = fma(b, v, nb);
+        b = nb;
+    } else if (j == 1) {
+        b = fma(b, v, p);
+        d = fma(d, v, b);
+    } else {
+        b = fma(b, v, p);
+    }
+}
+
+template <typename T, typename TO, int NI, int BX, int BY, int BZ>
+__global__ void __launch_bounds__(arbs3::SEP_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
+k_eval_fused3(ArbGeom g, ArbBuckets B, const double* __restrict__ vals,
+              const double* __restrict__ q, int64_t n, int64_t ldq, ArbOut o,
+              const int32_t* __restrict__ offs, const int32_t* __restrict__ perm,
+              const int32_t* __restrict__ hot) {
+    constexpr int TH = arbs3::SEP_THREADS, R = FUSED_ROWS;
+    constexpr int NX = BX + 3, NY = BY + 3, NZ = BZ + 3, NT = NX * NY * NZ, NC = BX * BY * BZ;
+    constexpr int PER = (NT + TH - 1) / TH;
+    constexpr bool COMPS = NI >= 3, NORM = NI != 3;
+    // doubles per (cell column, node plane) of t2: 16 values, padded so that
+    // neighbouring columns start in different banks
+    constexpr int CS = 18, PL = BX * BY * CS;
+    constexpr int POS = ARB_EVAL_CHUNK + NC + (NC & 1);    // sorted positions, gaps included
+    __shared__ double nodes[NT];
+    __shared__ __align__(16) double t2[NZ * PL];           // [z][cy][cx][4 ey + ex]
+    __shared__ double srow[3][POS];
+    __shared__ int32_t sidx[POS];
+    __shared__ unsigned char scell[POS / 2];
+    __shared__ unsigned char cbad[NC];                     // cells with a non-finite stencil
+    __shared__ int32_t ccount[NC], cbase[NC + 1];
     int64_t b;
     int32_t start, end;
     if (!bucket_rows(offs, B.nbt, hot, ARB_EVAL_CHUNK, &b, &start, &end)) return;
+    const int tid = threadIdx.x;
     int64_t c0[3];
-    {
-        int64_t rem = b;
+    bucket_origin<3>(b, B, c0);
+    // node values of one interpolant: element tid + j TH of the tile, x
+    // fastest.  Nodes past the grid edge read as 0 (only cells outside the
+    // grid use them); the loads are unconditional (index 0 when unused).
+    double nv[PER];
+    int64_t nsrc[PER];
+    bool nin[PER];
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            c0[a] = (rem % B.nb[a]) << B.bsh[a];
-            rem /= B.nb[a];
-        }
-    }
-    constexpr int NX = BX + 3, NY = BY + 3, NT = NX * NY * (BZ + 3);
-    double* nodes = reinterpret_cast<double*>(smem + B.ncell * B.cellstride);
-    double* t1 = nodes + NT;
-    double* t2 = t1 + arbs3::sep3_t1(BX, BY, BZ);
-    T* cf = reinterpret_cast<T*>(smem);
-    const int cstr = B.cellstride * (16 / (int)sizeof(T));   // elements per LDS cell
-    // this thread's first query, loaded before the coefficient work
-    int32_t s = start + threadIdx.x;
-    int64_t qi = -1;
-    double qp[3];
-    if (s < end) {
-        const int64_t pi = perm[s];
-        qi = (pi >= 0 && pi < n) ? pi : -1;         // always in range: perm holds row indices
-        const int64_t qq = qi >= 0 ? qi : 0;
-#pragma unroll
-        for (int a = 0; a < 3; ++a) qp[a] = q[qq * ldq + a];
-    }
-    // node tiles of every interpolant, x fastest: element e = k * NT + r of
-    // the flattened [interp][tile] space sits in register j of thread
-    // e - j * blockDim.x (the launcher checks ninterp * NT <= FUSED_REGS *
-    // blockDim.x).  Nodes past the grid edge read as 0 (only cells outside
-    // the grid use them); the loads are unconditional (index 0 when unused).
-    double nv[FUSED_REGS];
-    const int total = ninterp * NT;
-#pragma unroll
-    for (int j = 0; j < FUSED_REGS; ++j) {
-        const int e = threadIdx.x + j * blockDim.x;
-        const int k = e / NT, r = e - k * NT;
-        const int x = r % NX, y = (r / NX) % NY, z = r / (NX * NY);
+    for (int j = 0; j < PER; ++j) {
+        const int e = tid + j * TH;
+        const int x = e % NX, y = (e / NX) % NY, z = e / (NX * NY);
         const int64_t nx = c0[0] + x, ny = c0[1] + y, nz = c0[2] + z;
-        const bool in = e < total && nx < g.n[0] && ny < g.n[1] && nz < g.n[2];
-        const int64_t src = in ? (int64_t)k * g.nnodes + nx + g.nstride[1] * ny + g.nstride[2] * nz
-                               : 0;
-        const double v = vals[src];
-        nv[j] = in ? v : 0.0;
+        nin[j] = e < NT && nx < g.n[0] && ny < g.n[1] && nz < g.n[2];
+        nsrc[j] = nin[j] ? nx + g.nstride[1] * ny + g.nstride[2] * nz : 0;
     }
-    __shared__ unsigned char cbad[BX * BY * BZ];        // cells with a non-finite stencil
-    for (int k = 0; k < ninterp; ++k) {
-        // tile k into LDS: the x pass of interpolant k - 1, the last reader
-        // of `nodes`, ended at that interpolant's first pass barrier (so did
-        // its last reader of cbad, the z pass's stores)
-        int nonfinite = 0;
+    auto load_nodes = [&](int k) {
+        const double* vk = vals + (int64_t)k * g.nnodes;
 #pragma unroll
-        for (int j = 0; j < FUSED_REGS; ++j) {
-            const int e = threadIdx.x + j * blockDim.x - k * NT;
-            if (e >= 0 && e < NT) {
-                nodes[e] = nv[j];
-                nonfinite |= !isfinite(nv[j]);
+        for (int j = 0; j < PER; ++j) {
+            const double v = vk[nsrc[j]];
+            nv[j] = nin[j] ? v : 0.0;
+        }
+    };
+    // the rows in cell order, each cell from an even position
+    {
+        int32_t qi[R];
+        double qp[R][3];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int32_t s = start + tid + r * TH;
+            qi[r] = s < end ? perm[s] : -1;
+            if (qi[r] >= n) qi[r] = -1;                    // unreachable: perm holds row indices
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int64_t qq = qi[r] >= 0 ? qi[r] : 0;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) qp[r][a] = q[qq * ldq + a];
+        }
+        load_nodes(0);
+        for (int i = tid; i < POS; i += TH) sidx[i] = -1;
+        for (int i = tid; i < NC; i += TH) ccount[i] = 0;
+        __syncthreads();
+        double loc[R][3];
+        int lc[R], rank[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (!local_cell<BX, BY, BZ>(qp[r], g, c0, loc[r], &lc[r])) {
+                // beside the block: an aliased index (a coordinate at IntMax)
+                int64_t ia[3];
+                bool oob;
+                const int64_t flat = arb_reduce_axes<3>(qp[r], g, loc[r], ia, &oob);
+                const int64_t bb = bucket_of<3>(flat, ia, g, B, &lc[r]);
+                // a row of another bucket cannot happen (same reduction as k_keys)
+                if (bb != b || flat >= g.nc || lc[r] >= NC) qi[r] = -1;
+            }
+            rank[r] = qi[r] >= 0 ? atomicAdd(&ccount[lc[r]], 1) : 0;
+        }
+        __syncthreads();
+        if (tid < 64) {                                    // items per cell, scanned
+            int carry = 0;
+            for (int i0 = 0; i0 < NC; i0 += 64) {
+                const int i = i0 + tid;
+                const int c = i < NC ? (ccount[i] + 1) >> 1 : 0;
+                int x = c;
+#pragma unroll
+                for (int d = 1; d < 64; d <<= 1) {
+                    const int y = __shfl_up(x, d);
+                    if (tid >= d) x += y;
+                }
+                if (i < NC) cbase[i] = carry + x - c;
+                carry += __shfl(x, 63);
+            }
+            if (tid == 0) cbase[NC] = carry;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (qi[r] < 0) continue;
+            const int p = 2 * cbase[lc[r]] + rank[r];
+#pragma unroll
+            for (int a = 0; a < 3; ++a) srow[a][p] = loc[r][a];
+            sidx[p] = qi[r];
+            if ((rank[r] & 1) == 0) scell[p >> 1] = (unsigned char)lc[r];
+        }
+        __syncthreads();
+    }
+    const int nitems = cbase[NC];
+    // one round unless the rows are so spread that their items exceed the
+    // threads (each round forms the passes again)
+    for (int i0 = 0; i0 < nitems; i0 += TH) {
+        const int item = i0 + tid;
+        const bool live = item < nitems;
+        constexpr int NO = (COMPS ? 3 : 0) + (NORM ? 4 : 0);
+        TO rec[2][NO];
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+            for (int i = 0; i < NO; ++i) rec[r][i] = (TO)0;
+        if (i0 > 0) load_nodes(0);
+#pragma unroll 1
+        for (int k = 0; k < NI; ++k) {
+            // the thread's and the item's places are formed again for every
+            // interpolant (opaque to the compiler), not held in registers
+            int t0 = threadIdx.x, it = item;
+            asm volatile("" : "+v"(t0), "+v"(it));
+            int nonfinite = 0;
+#pragma unroll
+            for (int j = 0; j < PER; ++j) {
+                const int e = t0 + j * TH;
+                if (e < NT) {
+                    nodes[e] = nv[j];
+                    nonfinite |= !isfinite(nv[j]);
+                }
+            }
+            // (every lane has evaluated interpolant k - 1)
+            const bool anybad = __syncthreads_or(nonfinite) != 0;
+            if (k + 1 < NI) load_nodes(k + 1);
+            if (anybad) arbs3::cell_bad3<BX, BY, BZ>(nodes, cbad);
+            // x and y passes of one (cell column, node plane) per thread; a
+            // row's x pass is formed again for the up to four columns in y that
+            // use it, which saves an LDS round trip and a barrier
+            for (int t = t0; t < BX * BY * NZ; t += TH) {
+                const int x = t % BX, y = (t / BX) % BY, z = t / (BX * BY);
+                double cxp[4][4];                          // [oy][ex]
+#pragma unroll
+                for (int oy = 0; oy < 4; ++oy) {
+                    const double* nd = nodes + (z * NY + y + oy) * NX + x;
+                    arbs3::cub4(nd[0], nd[1], nd[2], nd[3], cxp[oy]);
+                }
+                double* out = t2 + z * PL + (y * BX + x) * CS;
+#pragma unroll
+                for (int h = 0; h < 4; h += 2) {
+                    double ca[4], cb[4];
+                    arbs3::cub4(cxp[0][h], cxp[1][h], cxp[2][h], cxp[3][h], ca);
+                    arbs3::cub4(cxp[0][h + 1], cxp[1][h + 1], cxp[2][h + 1], cxp[3][h + 1], cb);
+#pragma unroll
+                    for (int ey = 0; ey < 4; ++ey)
+                        *reinterpret_cast<double2*>(out + 4 * ey + h) = make_double2(ca[ey], cb[ey]);
+                }
+            }
+            __syncthreads();
+            if (!live) continue;
+            const int lc = scell[it];
+            const int cx = lc % BX, cy = (lc / BX) % BY, cz = lc / (BX * BY);
+            const bool two = sidx[2 * it + 1] >= 0;
+            T u[2], v[2], w[2];
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                const int p = 2 * it + (two ? r : 0);
+                u[r] = (T)srow[0][p];
+                v[r] = (T)srow[1][p];
+                w[r] = (T)srow[2][p];
+            }
+            const bool bad = anybad && cbad[lc];
+            const double* col = t2 + cz * PL + (cy * BX + cx) * CS;
+            // the four coefficients (ez) of every ex, for one ey, two ex at a time
+            auto coef = [&](int ey, T (*al)[4]) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    double2 f[4];
+#pragma unroll
+                    for (int z = 0; z < 4; ++z)
+                        f[z] = *reinterpret_cast<const double2*>(col + z * PL + 4 * ey + 2 * h);
+                    double ca[4], cb[4];
+                    arbs3::cub4(f[0].x, f[1].x, f[2].x, f[3].x, ca);
+                    arbs3::cub4(f[0].y, f[1].y, f[2].y, f[3].y, cb);
+#pragma unroll
+                    for (int ez = 0; ez < 4; ++ez) {
+                        al[2 * h][ez] = anybad && bad ? (T)NAN : (T)ca[ez];
+                        al[2 * h + 1][ez] = anybad && bad ? (T)NAN : (T)cb[ez];
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+            if (NORM && k == NI - 1) {
+                T qv[2][4], qd[2][4], qu[2][4];
+#pragma unroll
+                for (int ey = 3; ey >= 0; --ey) {
+                    T al[4][4];
+                    coef(ey, al);
+#pragma unroll
+                    for (int r = 0; r < 2; ++r)
+#pragma unroll
+                        for (int ez = 0; ez < 4; ++ez) {
+                            T p, pu;
+                            h4d<T>(al[0][ez], al[1][ez], al[2][ez], al[3][ez], u[r], p, pu);
+                            stream_h4d<T>(ey, p, v[r], qv[r][ez], qd[r][ez]);
+                            stream_h4<T>(ey, pu, v[r], qu[r][ez]);
+                        }
+                }
+                constexpr int at = COMPS ? 3 : 0;
+#pragma unroll
+                for (int r = 0; r < 2; ++r) {
+                    T val, dw;
+                    h4d<T>(qv[r][0], qv[r][1], qv[r][2], qv[r][3], w[r], val, dw);
+                    const T gu = h4<T>(qu[r][0], qu[r][1], qu[r][2], qu[r][3], w[r]);
+                    const T gv = h4<T>(qd[r][0], qd[r][1], qd[r][2], qd[r][3], w[r]);
+                    rec[r][at] = (TO)val;
+                    rec[r][at + 1] = (TO)(gu / (T)g.h[0]);
+                    rec[r][at + 2] = (TO)(gv / (T)g.h[1]);
+                    rec[r][at + 3] = (TO)(dw / (T)g.h[2]);
+                }
+            } else {
+                T qv[2][4];
+#pragma unroll
+                for (int ey = 3; ey >= 0; --ey) {
+                    T al[4][4];
+                    coef(ey, al);
+#pragma unroll
+                    for (int r = 0; r < 2; ++r)
+#pragma unroll
+                        for (int ez = 0; ez < 4; ++ez)
+                            stream_h4<T>(ey, h4<T>(al[0][ez], al[1][ez], al[2][ez], al[3][ez], u[r]),
+                                         v[r], qv[r][ez]);
+                }
+#pragma unroll
+                for (int r = 0; r < 2; ++r) {
+                    const TO val = (TO)h4<T>(qv[r][0], qv[r][1], qv[r][2], qv[r][3], w[r]);
+                    rec[r][0] = k == 0 ? val : rec[r][0];
+                    rec[r][1] = k == 1 ? val : rec[r][1];
+                    rec[r][2] = k == 2 ? val : rec[r][2];
+                }
             }
         }
-        const bool anybad = __syncthreads_or(nonfinite) != 0;
-        if (anybad) {
-            arbs3::cell_bad3<BX, BY, BZ>(nodes, cbad);
-            __syncthreads();
-        }
-        // consecutive threads, consecutive cells: local cell cx + BX (cy + BY cz)
-        arbs3::sep3_passes<BX, BY, BZ, true>(nodes, t1, t2,
-                                             [&](int cx, int cy, int cz, int i, double a) {
-            const int lc = cx + BX * (cy + BY * cz);
-            if (anybad && cbad[lc]) a = NAN;
-            cf[lc * cstr + k * 64 + i] = (T)a;
-        });
-    }
-    __syncthreads();
-    if (qi >= 0) eval_row_lds<3, T, T, TO>(g, B, smem, has_comps, has_norm, o, b, qi, qp);
-    for (s += blockDim.x; s < end; s += blockDim.x) {
-        const int64_t pi = perm[s];
-        if (pi < 0 || pi >= n) continue;            // unreachable: perm holds row indices
 #pragma unroll
-        for (int a = 0; a < 3; ++a) qp[a] = q[pi * ldq + a];
-        eval_row_lds<3, T, T, TO>(g, B, smem, has_comps, has_norm, o, b, pi, qp);
+        for (int r = 0; r < 2; ++r) {
+            const int32_t i = live ? sidx[2 * item + r] : -1;
+            TO full[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) full[j] = j < NO ? rec[r][j] : (TO)0;
+            if (i >= 0) store_rec<3, TO>(full, COMPS, NORM, o, i);
+        }
     }
 }
 
@@ -968,14 +1206,7 @@ k_eval_fused4(ArbGeom g, ArbBuckets B, const double* __restrict__ vals, int32_t 
     int32_t start, end;
     if (!bucket_rows(offs, B.nbt, hot, ARB_EVAL_CHUNK, &b, &start, &end)) return;
     int64_t c0[4];
-    {
-        int64_t rem = b;
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            c0[a] = (rem % B.nb[a]) << B.bsh[a];
-            rem /= B.nb[a];
-        }
-    }
+    bucket_origin<4>(b, B, c0);
     double* nodes = reinterpret_cast<double*>(smem + B.ncell * B.cellstride);
     double* t3 = nodes + S::NT4;
     double* t1 = t3 + S::NT3;
@@ -1222,14 +1453,6 @@ struct TileShape {
 };
 
 // Tile origin (first cell = first node) of bucket b, per axis.
-__device__ __forceinline__ void bucket_origin3(int64_t b, const ArbBuckets& B, int64_t* c0) {
-    int64_t rem = b;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        c0[a] = (rem % B.nb[a]) << B.bsh[a];
-        rem /= B.nb[a];
-    }
-}
 
 // The model of interpolant k (values v = that interpolant's node values)
 // around grid node mi: F(mi) and the central first differences, and for the
@@ -1321,7 +1544,7 @@ k_build_tiles3(ArbGeom g, ArbBuckets B, const double* __restrict__ vals,
     __shared__ int best;
     const int64_t b = blockIdx.x;
     int64_t c0[3];
-    bucket_origin3(b, B, c0);
+    bucket_origin<3>(b, B, c0);
     // the centre range per axis: one node inside the grid so that the central
     // differences exist (two where the axis has 5 nodes or more, for the third
     // differences along it); the default centre is the tile's middle node
@@ -1963,55 +2186,46 @@ hipError_t arb_launch_eval_bucket(const ArbGeom& g, const ArbBuckets& B, int32_t
 // geometry is chosen from).
 #define ARB_FUSED_SHAPES(X) X(4, 4, 4) X(4, 4, 2) X(4, 2, 2) X(2, 2, 2) X(2, 2, 1) X(2, 1, 1) X(1, 1, 1)
 
-// LDS bytes of k_eval_fused3 for the bucket geometry B (0 when the path does
-// not apply: 3D only, an instantiated block shape, within 160 KiB, node tiles
-// of all interpolants within the registers of the workgroup).  The fused
-// kernels run arbs3::SEP_THREADS threads per workgroup whatever the tuning's
-// thread count (the separable passes stride by it).
-size_t arb_fused_lds(const ArbGeom& g, const ArbBuckets& B, int32_t ninterp, int32_t threads) {
-    (void)threads;
-    if (g.ndim != 3) return 0;
+// Whether k_eval_fused3 takes the bucket geometry B: 3D, an instantiated
+// block shape, the local cell index cx + bx (cy + by cz).  (The fused kernels
+// run arbs3::SEP_THREADS threads per workgroup whatever the tuning's thread
+// count: the separable passes stride by it.)
+bool arb_fused_ok(const ArbGeom& g, const ArbBuckets& B, int32_t ninterp) {
+    if (g.ndim != 3 || (ninterp != 1 && ninterp != 3 && ninterp != 4)) return false;
     const int bx = B.b[0], by = B.b[1], bz = B.b[2];
     bool shape = false;
 #define ARB_FUSED_IS(X, Y, Z) shape |= (bx == X && by == Y && bz == Z);
     ARB_FUSED_SHAPES(ARB_FUSED_IS)
 #undef ARB_FUSED_IS
-    if (!shape) return 0;
-    // the local cell index must be cx + bx (cy + by cz), as the kernel writes it
-    if (B.lsh[0] != 0 || (1 << B.lsh[1]) != bx || (1 << B.lsh[2]) != bx * by) return 0;
-    if ((int64_t)ninterp * arbs3::sep3_nodes(bx, by, bz) > (int64_t)FUSED_REGS * arbs3::SEP_THREADS)
-        return 0;
-    const size_t lds = (size_t)B.ncell * B.cellstride * 16 +
-                       sizeof(double) * (size_t)(arbs3::sep3_nodes(bx, by, bz) +
-                                                 arbs3::sep3_t1(bx, by, bz) +
-                                                 arbs3::sep3_t2(bx, by, bz));
-    // gfx950: 160 KiB of LDS per workgroup, with room for the kernel's static
-    // LDS (one byte per cell)
-    return lds + 256 <= 160 * 1024 ? lds : 0;
+    return shape && B.lsh[0] == 0 && (1 << B.lsh[1]) == bx && (1 << B.lsh[2]) == bx * by;
 }
 
 hipError_t arb_launch_eval_fused(const ArbGeom& g, const ArbBuckets& B, int32_t prec,
                                  int32_t out_f64, const double* vals, int32_t ninterp,
-                                 int32_t has_comps, int32_t has_norm, const double* q, int64_t n,
-                                 int64_t ldq, const ArbOut& o, const int32_t* offs,
-                                 const int32_t* perm, const int32_t* hot, int32_t block_threads,
+                                 const double* q, int64_t n, int64_t ldq, const ArbOut& o,
+                                 const int32_t* offs, const int32_t* perm, const int32_t* hot,
                                  hipStream_t s) {
-    (void)block_threads;
-    const size_t lds = arb_fused_lds(g, B, ninterp, arbs3::SEP_THREADS);
-    if (lds == 0) return hipErrorInvalidValue;
+    if (!arb_fused_ok(g, B, ninterp)) return hipErrorInvalidValue;
     dim3 grid(eval_grid(B, n)), block(arbs3::SEP_THREADS);
-#define L_FUSED(T, TO, X, Y, Z)                                                               \
-    hipLaunchKernelGGL((k_eval_fused3<T, TO, X, Y, Z>), grid, block, lds, s, g, B, vals,      \
-                       ninterp, has_comps, has_norm, q, n, ldq, o, offs, perm, hot)
+#define L_FUSED(T, TO, NI, X, Y, Z)                                                           \
+    hipLaunchKernelGGL((k_eval_fused3<T, TO, NI, X, Y, Z>), grid, block, 0, s, g, B, vals, q,  \
+                       n, ldq, o, offs, perm, hot)
+#define L_FUSED_NI(NI, X, Y, Z)                                                               \
+    {                                                                                         \
+        if (prec == ARB_PREC_FP64) L_FUSED(double, double, NI, X, Y, Z);                      \
+        else if (out_f64) L_FUSED(float, double, NI, X, Y, Z);                                \
+        else L_FUSED(float, float, NI, X, Y, Z);                                              \
+    }
 #define ARB_FUSED_CASE(X, Y, Z)                                                               \
     if (B.b[0] == X && B.b[1] == Y && B.b[2] == Z) {                                          \
-        if (prec == ARB_PREC_FP64) L_FUSED(double, double, X, Y, Z);                          \
-        else if (out_f64) L_FUSED(float, double, X, Y, Z);                                    \
-        else L_FUSED(float, float, X, Y, Z);                                                  \
+        if (ninterp == 4) L_FUSED_NI(4, X, Y, Z)                                              \
+        else if (ninterp == 3) L_FUSED_NI(3, X, Y, Z)                                         \
+        else L_FUSED_NI(1, X, Y, Z)                                                           \
         return hipGetLastError();                                                             \
     }
     ARB_FUSED_SHAPES(ARB_FUSED_CASE)
 #undef ARB_FUSED_CASE
+#undef L_FUSED_NI
 #undef L_FUSED
     return hipErrorInvalidValue;
 }
