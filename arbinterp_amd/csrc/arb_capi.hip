@@ -2,6 +2,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdarg>
+#include <cstddef>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -191,23 +192,14 @@ struct arb_field {
     ArbBuckets BF{};
     int32_t user_block[ARB_MAXD] = {0, 0, 0, 0};
     int32_t eval_threads = 256;
-    int32_t* ws_bkt = nullptr;  // per query: bucket (-1 = handled in place)
-    int32_t* ws_rank = nullptr; // per query: rank inside its bucket
-    int32_t* ws_perm = nullptr; // bucket-sorted query indices
+    void* ws = nullptr;         // sort workspace (carve_sort_ws), one allocation
+    int64_t ws_bytes = 0;
+    int32_t* ws_group = nullptr; // ARB_Q_GROUP_ATOMIC: bucket, rank and position per query
+    int64_t ws_group_n = 0;
     void* ws_rec = nullptr;     // packed output records of a bucketed call (split afterwards)
     int64_t ws_rec_bytes = 0;
     void* ws_qrec = nullptr;    // per-row records of the node-tile path (16 bytes per row)
     int64_t ws_qrec_n = 0;
-    int64_t ws_n = 0;
-    int32_t* ws_count = nullptr;
-    int32_t* ws_offs = nullptr;
-    int64_t ws_nb = 0;
-    // radix-sort workspace: keys/values x2, digit histograms, scan temporaries
-    uint32_t* rs_k[2] = {nullptr, nullptr};
-    int32_t* rs_v[2] = {nullptr, nullptr};
-    int32_t* rs_hist = nullptr;    // tile digit histograms
-    int32_t* rs_hscan = nullptr;   // their per-digit scans, then the digit totals
-    int64_t rs_n = 0;
     // backward workspace
     int32_t* bw_key = nullptr;     // per query: cell (nc outside)
     int32_t* bw_perm = nullptr;    // queries grouped per cell, index order
@@ -311,50 +303,6 @@ static void choose_buckets(arb_field* f, ArbBuckets& B, bool table) {
         B.ncell *= B.b[a];
         B.nbt *= B.nb[a];
     }
-}
-
-static int ensure_workspace(arb_field* f, int64_t n, int64_t nbt) {
-    if (n > f->ws_n) {
-        if (f->ws_bkt) (void)hipFree(f->ws_bkt);
-        if (f->ws_rank) (void)hipFree(f->ws_rank);
-        if (f->ws_perm) (void)hipFree(f->ws_perm);
-        f->ws_bkt = f->ws_rank = f->ws_perm = nullptr;
-        f->ws_n = 0;
-        HIPCHK(hipMalloc(&f->ws_bkt, sizeof(int32_t) * n));
-        HIPCHK(hipMalloc(&f->ws_rank, sizeof(int32_t) * n));
-        HIPCHK(hipMalloc(&f->ws_perm, sizeof(int32_t) * n));
-        f->ws_n = n;
-    }
-    if (n > f->rs_n) {
-        for (int k = 0; k < 2; ++k) {
-            if (f->rs_k[k]) (void)hipFree(f->rs_k[k]);
-            if (f->rs_v[k]) (void)hipFree(f->rs_v[k]);
-            f->rs_k[k] = nullptr;
-            f->rs_v[k] = nullptr;
-        }
-        if (f->rs_hist) (void)hipFree(f->rs_hist);
-        if (f->rs_hscan) (void)hipFree(f->rs_hscan);
-        f->rs_hist = f->rs_hscan = nullptr;
-        f->rs_n = 0;
-        const int64_t hl = 256 * arb_rs_ntiles(n);
-        for (int k = 0; k < 2; ++k) {
-            HIPCHK(hipMalloc(&f->rs_k[k], sizeof(uint32_t) * n));
-            HIPCHK(hipMalloc(&f->rs_v[k], sizeof(int32_t) * n));
-        }
-        HIPCHK(hipMalloc(&f->rs_hist, sizeof(int32_t) * hl));
-        HIPCHK(hipMalloc(&f->rs_hscan, sizeof(int32_t) * (hl + 256)));   // + digit totals
-        f->rs_n = n;
-    }
-    if (nbt + 1 > f->ws_nb) {
-        if (f->ws_count) (void)hipFree(f->ws_count);
-        if (f->ws_offs) (void)hipFree(f->ws_offs);
-        f->ws_count = f->ws_offs = nullptr;
-        f->ws_nb = 0;
-        HIPCHK(hipMalloc(&f->ws_count, sizeof(int32_t) * arb_rs_first_elems(nbt)));
-        HIPCHK(hipMalloc(&f->ws_offs, sizeof(int32_t) * (nbt + 1)));
-        f->ws_nb = nbt + 1;
-    }
-    return ARB_OK;
 }
 
 // Per-row records of the node-tile bucketed path (n x 16 bytes), made on
@@ -485,35 +433,59 @@ int arb_field_create(const double* rows_dev, int64_t nrows, int32_t ncols, int64
     HIPCHK(hipMalloc(&f->flag, sizeof(int32_t) * 4));
     HIPCHK(hipMemsetAsync(f->flag, 0, sizeof(int32_t) * 4, s));
 
-    // 1. coordinates must be finite
-    HIPCHK(arb_launch_finite_check(rows_dev, nrows, ncols, ld, ndim, f->flag, s));
-    int32_t hflag = 0;
-    HIPCHK(hipMemcpyAsync(&hflag, f->flag, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
-    if (hflag) return fail(ARB_EGRID, "field has a non-finite coordinate");
-
-    // 2. unique values per axis
-    int64_t cap = 1024;
-    while (cap < 2 * nrows) cap <<= 1;
-    DevBuf tab, uniq, cnt;
-    HIPCHK(tab.alloc(sizeof(unsigned long long) * cap));
-    HIPCHK(uniq.alloc(sizeof(double) * cap));
-    HIPCHK(cnt.alloc(sizeof(unsigned int)));
+    // 1. unique values per axis (and that coordinates are finite): one pass
+    // over the rows into small hash sets, their values listed as they are
+    // found; one copy back, a second one only for axes of more than AXES_FEW
+    // values.  An axis of more than AXES_MAX takes hash sets sized for any
+    // rows, an axis at a time.
     std::vector<std::vector<double>> axes(ndim);
-    for (int a = 0; a < ndim; ++a) {
-        HIPCHK(hipMemsetAsync(tab.p, 0xFF, sizeof(unsigned long long) * cap, s));
-        HIPCHK(hipMemsetAsync(cnt.p, 0, sizeof(unsigned int), s));
-        HIPCHK(arb_launch_hash_insert(rows_dev, nrows, ld, a, tab.as<unsigned long long>(), cap, s));
-        HIPCHK(arb_launch_hash_compact(tab.as<unsigned long long>(), cap, uniq.as<double>(),
-                                       cnt.as<unsigned int>(), s));
-        unsigned int nu = 0;
-        HIPCHK(hipMemcpyAsync(&nu, cnt.p, sizeof nu, hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
-        axes[a].resize(nu);
-        HIPCHK(hipMemcpyAsync(axes[a].data(), uniq.p, sizeof(double) * nu, hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
-        std::sort(axes[a].begin(), axes[a].end());
+    DevBuf sets;
+    HIPCHK(sets.alloc(arb_axes_bytes(ndim)));
+    const AxesLayout L = arb_axes_layout(sets.p, ndim);
+    HIPCHK(hipMemsetAsync(L.hash, 0xFF, L.hash_bytes, s));
+    HIPCHK(hipMemsetAsync(L.head, 0, sizeof(AxesHead), s));
+    HIPCHK(arb_launch_axes(rows_dev, nrows, ld, ndim, L, s));
+    struct { AxesHead head; double few[ARB_MAXD * AXES_FEW]; } got;
+    static_assert(offsetof(decltype(got), few) == sizeof(AxesHead), "the head, then the values");
+    HIPCHK(hipMemcpyAsync(&got, L.head, sizeof(AxesHead) + sizeof(double) * ndim * AXES_FEW,
+                          hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    if (got.head.nonfinite) return fail(ARB_EGRID, "field has a non-finite coordinate");
+    if (!got.head.overflow) {
+        for (int a = 0; a < ndim; ++a) {
+            const int64_t nu = got.head.count[a], few = nu < AXES_FEW ? nu : (int64_t)AXES_FEW;
+            axes[a].assign(got.few + a * AXES_FEW, got.few + a * AXES_FEW + few);
+            if (nu > few) {
+                axes[a].resize(nu);
+                HIPCHK(hipMemcpyAsync(axes[a].data() + few, L.more + (int64_t)a * AXES_MAX,
+                                      sizeof(double) * (nu - few), hipMemcpyDeviceToHost, s));
+                HIPCHK(hipStreamSynchronize(s));
+            }
+        }
+    } else {
+        int64_t cap = 1024;
+        while (cap < 2 * nrows) cap <<= 1;
+        DevBuf tab, uniq, cnt;
+        HIPCHK(tab.alloc(sizeof(unsigned long long) * cap));
+        HIPCHK(uniq.alloc(sizeof(double) * cap));
+        HIPCHK(cnt.alloc(sizeof(unsigned int)));
+        for (int a = 0; a < ndim; ++a) {
+            HIPCHK(hipMemsetAsync(tab.p, 0xFF, sizeof(unsigned long long) * cap, s));
+            HIPCHK(hipMemsetAsync(cnt.p, 0, sizeof(unsigned int), s));
+            HIPCHK(arb_launch_hash_insert(rows_dev, nrows, ld, a, tab.as<unsigned long long>(),
+                                          cap, s));
+            HIPCHK(arb_launch_hash_compact(tab.as<unsigned long long>(), cap, uniq.as<double>(),
+                                           cnt.as<unsigned int>(), s));
+            unsigned int nu = 0;
+            HIPCHK(hipMemcpyAsync(&nu, cnt.p, sizeof nu, hipMemcpyDeviceToHost, s));
+            HIPCHK(hipStreamSynchronize(s));
+            axes[a].resize(nu);
+            HIPCHK(hipMemcpyAsync(axes[a].data(), uniq.p, sizeof(double) * nu,
+                                  hipMemcpyDeviceToHost, s));
+            HIPCHK(hipStreamSynchronize(s));
+        }
     }
+    for (auto& v : axes) std::sort(v.begin(), v.end());
     ArbGeom& g = f->g;
     g.ndim = ndim;
     int64_t prod = 1;
@@ -547,26 +519,29 @@ int arb_field_create(const double* rows_dev, int64_t nrows, int32_t ncols, int64
     if (g.nc >= ((int64_t)1 << 32))
         return fail(ARB_EGRID, "grid too large: %lld cells (limit 2^32)", (long long)g.nc);
 
-    // 3. rank rows, scatter values into canonical order, check completeness
-    DevBuf axes_dev[ARB_MAXD], seen;
+    // 2. rank rows, scatter values into canonical order, check that every node
+    // was written (with as many rows as nodes, then each exactly once)
+    DevBuf axbuf, seen;
+    std::vector<double> axall;
     const double* axp[ARB_MAXD] = {nullptr, nullptr, nullptr, nullptr};
-    for (int a = 0; a < ndim; ++a) {
-        HIPCHK(axes_dev[a].alloc(sizeof(double) * g.n[a]));
-        HIPCHK(hipMemcpyAsync(axes_dev[a].p, axes[a].data(), sizeof(double) * g.n[a],
-                              hipMemcpyHostToDevice, s));
-        axp[a] = axes_dev[a].as<double>();
-    }
-    HIPCHK(seen.alloc(sizeof(int32_t) * g.nnodes));
-    HIPCHK(hipMemsetAsync(seen.p, 0, sizeof(int32_t) * g.nnodes, s));
+    for (int a = 0; a < ndim; ++a) axall.insert(axall.end(), axes[a].begin(), axes[a].end());
+    HIPCHK(axbuf.alloc(sizeof(double) * axall.size()));
+    HIPCHK(hipMemcpyAsync(axbuf.p, axall.data(), sizeof(double) * axall.size(),
+                          hipMemcpyHostToDevice, s));
+    for (int64_t a = 0, at = 0; a < ndim; at += g.n[a++]) axp[a] = axbuf.as<double>() + at;
+    const int64_t seen_bytes = (g.nnodes + 7) / 8 * 8;
+    HIPCHK(seen.alloc(seen_bytes));
+    HIPCHK(hipMemsetAsync(seen.p, 0, seen_bytes, s));
     HIPCHK(hipMalloc(&f->vals, sizeof(double) * g.nnodes * f->ninterp));
     HIPCHK(arb_launch_rank_scatter(rows_dev, nrows, ld, axp, g, mode | f32_norm, ndim, f->vals,
-                                   f->ninterp, seen.as<int32_t>(), s));
-    HIPCHK(arb_launch_check_seen(seen.as<int32_t>(), g.nnodes, f->flag, s));
+                                   seen.as<unsigned char>(), s));
+    HIPCHK(arb_launch_check_seen(seen.as<unsigned char>(), g.nnodes, f->flag, s));
+    int32_t hflag = 0;
     HIPCHK(hipMemcpyAsync(&hflag, f->flag, sizeof(int32_t), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
     if (hflag) return fail(ARB_EGRID, "rows do not form a complete grid (duplicate points)");
 
-    // 4. table size and the sentinel row
+    // 3. table size and the sentinel row
     const int K = 1 << (2 * ndim);
     const size_t esz = precision == ARB_PREC_FP64 ? sizeof(double) : sizeof(float);
     // the table itself is allocated by its first build (node-tile queries
@@ -777,6 +752,34 @@ static int64_t carve_sort_ws(unsigned char* base, int64_t n, int64_t nbt, bool q
     return off;
 }
 
+// The field's own sort workspace for n rows and nbt buckets, grown when a call
+// needs more: one allocation (a hipMalloc and its hipFree cost a new field
+// about 25 us, and eight buffers were allocated apart).
+static int ensure_workspace(arb_field* f, int64_t n, int64_t nbt, SortWs* w) {
+    const int64_t need = carve_sort_ws(nullptr, n, nbt, false, w);
+    if (need > f->ws_bytes) {
+        if (f->ws) (void)hipFree(f->ws);
+        f->ws = nullptr;
+        f->ws_bytes = 0;
+        HIPCHK(hipMalloc(&f->ws, (size_t)need));
+        f->ws_bytes = need;
+    }
+    carve_sort_ws(static_cast<unsigned char*>(f->ws), n, nbt, false, w);
+    return ARB_OK;
+}
+
+// Bucket, rank and position per query (ARB_Q_GROUP_ATOMIC), made on first use.
+static int ensure_group(arb_field* f, int64_t n) {
+    if (n > f->ws_group_n) {
+        if (f->ws_group) (void)hipFree(f->ws_group);
+        f->ws_group = nullptr;
+        f->ws_group_n = 0;
+        HIPCHK(hipMalloc(&f->ws_group, sizeof(int32_t) * 3 * n));
+        f->ws_group_n = n;
+    }
+    return ARB_OK;
+}
+
 // arb_query and arb_query_noalloc.  With noalloc the call allocates nothing:
 // the table or node tiles must already be allocated (they are rebuilt in
 // place when the node values changed), the bucketed path takes its sort
@@ -936,16 +939,8 @@ static int query_impl(arb_field* f, double* q_dev, int64_t n, int64_t ldq, void*
                             (long long)need, (long long)ARB_NOALLOC_SCRATCH_BYTES);
             carve_sort_ws(base, n, BB.nbt, nodeform, &w);
         } else {
-            rc = ensure_workspace(f, n, BB.nbt);
+            rc = ensure_workspace(f, n, BB.nbt, &w);
             if (rc) return rc;
-            for (int k = 0; k < 2; ++k) {
-                w.k[k] = f->rs_k[k];
-                w.v[k] = f->rs_v[k];
-            }
-            w.hist = f->rs_hist;
-            w.hscan = f->rs_hscan;
-            w.first = f->ws_count;
-            w.offs = f->ws_offs;
         }
         // separate output arrays of a 3D field: the bucketed kernels write
         // each row as one packed record into the workspace, and k_unpack
@@ -989,21 +984,25 @@ static int query_impl(arb_field* f, double* q_dev, int64_t n, int64_t ldq, void*
                 w.qrec = f->ws_qrec;
             }
         }
-        const int32_t* perm = f->ws_perm;
+        const int32_t* perm = nullptr;
         // the evaluation's hot flag (a bucket holds more rows than one
         // workgroup takes): the last int of w.first, set by the grouping
         // sort, and set to 1 (look) by the other groupings
         int32_t* hot = w.first + arb_rs_first_elems(BB.nbt) - 1;
         if (timing) HIPCHK(hipEventRecord(f->ev[0], s));
         if (flags & ARB_Q_GROUP_ATOMIC) {
-            HIPCHK(arb_launch_fill_i32(f->ws_count, f->B.nbt, 0, s));
+            rc = ensure_group(f, n);
+            if (rc) return rc;
+            int32_t *bkt = f->ws_group, *rank = bkt + n, *place = rank + n;
+            HIPCHK(arb_launch_fill_i32(w.first, f->B.nbt, 0, s));
             HIPCHK(arb_launch_bucket(f->g, f->B, f->precision, out64, f->table, f->ninterp,
-                                     f->has_comps, f->has_norm, q_dev, n, ldq, o, f->ws_bkt,
-                                     f->ws_rank, f->ws_count, s));
+                                     f->has_comps, f->has_norm, q_dev, n, ldq, o, bkt, rank,
+                                     w.first, s));
             if (timing) HIPCHK(hipEventRecord(f->ev[1], s));
-            HIPCHK(arb_launch_scan(f->ws_count, f->ws_offs, f->B.nbt, s));
+            HIPCHK(arb_launch_scan(w.first, w.offs, f->B.nbt, s));
             if (timing) HIPCHK(hipEventRecord(f->ev[2], s));
-            HIPCHK(arb_launch_scatter(f->ws_bkt, f->ws_rank, f->ws_offs, f->ws_perm, n, s));
+            HIPCHK(arb_launch_scatter(bkt, rank, w.offs, place, n, s));
+            perm = place;
             HIPCHK(arb_launch_fill_i32(hot, 1, 1, s));
         } else {
             // key = bucket (then the cell inside it with ARB_Q_SORT_CELL)
@@ -1612,19 +1611,10 @@ void arb_field_destroy(arb_field* f) {
     if (f->table) (void)hipFree(f->table);
     if (f->sent) (void)hipFree(f->sent);
     if (f->flag) (void)hipFree(f->flag);
-    if (f->ws_bkt) (void)hipFree(f->ws_bkt);
-    if (f->ws_rank) (void)hipFree(f->ws_rank);
-    if (f->ws_perm) (void)hipFree(f->ws_perm);
+    if (f->ws) (void)hipFree(f->ws);
+    if (f->ws_group) (void)hipFree(f->ws_group);
     if (f->ws_rec) (void)hipFree(f->ws_rec);
     if (f->ws_qrec) (void)hipFree(f->ws_qrec);
-    if (f->ws_count) (void)hipFree(f->ws_count);
-    if (f->ws_offs) (void)hipFree(f->ws_offs);
-    for (int k = 0; k < 2; ++k) {
-        if (f->rs_k[k]) (void)hipFree(f->rs_k[k]);
-        if (f->rs_v[k]) (void)hipFree(f->rs_v[k]);
-    }
-    if (f->rs_hist) (void)hipFree(f->rs_hist);
-    if (f->rs_hscan) (void)hipFree(f->rs_hscan);
     if (f->bw_key) (void)hipFree(f->bw_key);
     if (f->bw_perm) (void)hipFree(f->bw_perm);
     if (f->bw_k1) (void)hipFree(f->bw_k1);

@@ -256,17 +256,37 @@ __device__ __forceinline__ void arb_valgrad4(const C* a, T u, T v, T w, T t, T& 
 // ---------------------------------------------------------------------------
 struct ArbField;
 
-hipError_t arb_launch_finite_check(const double* rows, int64_t nrows, int32_t ncols, int64_t ld,
-                                   int32_t ndim, int32_t* flag, hipStream_t s);
+// Unique coordinates per axis of the field's rows (k_grid.hip): per axis a
+// hash set of AXES_SLOTS slots that takes up to AXES_MAX values, and the list
+// of its values: the first AXES_FEW of every axis behind the head, the others
+// apart.
+constexpr int AXES_SLOTS = 65536, AXES_MAX = AXES_SLOTS / 2, AXES_FEW = 1024;
+struct AxesHead {
+    uint32_t count[ARB_MAXD];
+    int32_t nonfinite, overflow;       // a non-finite coordinate; an axis past AXES_MAX
+};
+struct AxesLayout {
+    unsigned long long* hash;          // [axis][AXES_SLOTS], 0xFF.. = empty
+    int64_t hash_bytes;
+    AxesHead* head;
+    double* few;                       // [axis][AXES_FEW]
+    double* more;                      // [axis][AXES_MAX]: values AXES_FEW and on
+};
+int64_t arb_axes_bytes(int32_t ndim);
+AxesLayout arb_axes_layout(void* base, int32_t ndim);
+hipError_t arb_launch_axes(const double* rows, int64_t nrows, int64_t ld, int32_t ndim,
+                           const AxesLayout& L, hipStream_t s);
 hipError_t arb_launch_hash_insert(const double* rows, int64_t nrows, int64_t ld, int32_t axis,
                                   unsigned long long* tab, int64_t cap, hipStream_t s);
 hipError_t arb_launch_hash_compact(const unsigned long long* tab, int64_t cap, double* out,
                                    unsigned int* count, hipStream_t s);
 hipError_t arb_launch_rank_scatter(const double* rows, int64_t nrows, int64_t ld,
                                    const double* const* axes_dev, const ArbGeom& g,
-                                   int32_t mode, int32_t vcol0, double* vals, int32_t ninterp,
-                                   int32_t* seen, hipStream_t s);
-hipError_t arb_launch_check_seen(const int32_t* seen, int64_t nnodes, int32_t* flag, hipStream_t s);
+                                   int32_t mode, int32_t vcol0, double* vals,
+                                   unsigned char* seen, hipStream_t s);
+// seen: one byte per node, padded to a multiple of eight.
+hipError_t arb_launch_check_seen(const unsigned char* seen, int64_t nnodes, int32_t* flag,
+                                 hipStream_t s);
 // Extend the node values src ([ninterp][go.nnodes]) to the grid gn (one ghost
 // layer per face) in dst ([ninterp][gn.nnodes]) with boundary rule bc.
 hipError_t arb_launch_pad_boundary(const double* src, const ArbGeom& go, double* dst,
