@@ -9,6 +9,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "arb_internal.h"
@@ -36,15 +37,148 @@ static int fail(int code, const char* fmt, ...) {
                         "%s failed: %s", #x, hipGetErrorString(e_));              \
     } while (0)
 
+// ---------------------------------------------------------------------------
+// Device memory.  Blocks of up to POOL_BLOCK bytes come back to a pool of at
+// most POOL_BYTES for the whole process (the oldest leave first, and all of
+// them when an allocation fails), so a program that makes one field after
+// another (a field per time step) does not pay for mapping and unmapping its
+// node values and workspaces each time: 112 x 96 x 88 nodes and 10^6 queries,
+// hipFree alone took 1.3 of 1.9 ms.  Larger blocks (tables) are freed at once.
+// A block enters the pool when its device is idle (as hipFree waits for it to
+// be), so whatever thread or stream takes it next, nothing still uses it.
+// ---------------------------------------------------------------------------
+namespace {
+
+constexpr size_t POOL_BLOCK = (size_t)128 << 20, POOL_BYTES = (size_t)512 << 20;
+constexpr size_t POOL_GRAIN = (size_t)64 << 10;
+
+struct DevPool {
+    struct Block {
+        void* p;
+        size_t bytes;
+        int dev;
+    };
+    std::mutex mu;
+    std::vector<Block> cached;                       // oldest first
+    std::unordered_map<void*, Block> used;
+    size_t held = 0;
+
+    hipError_t take(void** out, size_t bytes) {
+        *out = nullptr;
+        int dev = 0;
+        hipError_t e = hipGetDevice(&dev);
+        if (e != hipSuccess) return e;
+        const size_t need = (bytes ? bytes + POOL_GRAIN - 1 : POOL_GRAIN) / POOL_GRAIN * POOL_GRAIN;
+        std::lock_guard<std::mutex> lock(mu);
+        size_t best = cached.size();
+        for (size_t i = 0; i < cached.size(); ++i)
+            if (cached[i].dev == dev && cached[i].bytes >= need &&
+                cached[i].bytes <= need + need / 4 + POOL_GRAIN &&
+                (best == cached.size() || cached[i].bytes < cached[best].bytes))
+                best = i;
+        Block b{nullptr, need, dev};
+        if (best < cached.size()) {
+            b = cached[best];
+            cached.erase(cached.begin() + (std::ptrdiff_t)best);
+            held -= b.bytes;
+        } else {
+            e = hipMalloc(&b.p, need);
+            if (e == hipErrorOutOfMemory && !cached.empty()) {
+                (void)hipGetLastError();
+                shrink(0);
+                e = hipMalloc(&b.p, need);
+            }
+            if (e != hipSuccess) return e;
+        }
+        try {
+            used.emplace(b.p, b);
+        } catch (...) {
+            (void)hipFree(b.p);
+            return hipErrorOutOfMemory;
+        }
+        *out = b.p;
+        return hipSuccess;
+    }
+
+    // idle: the block's device has been waited for (else it is freed, which waits)
+    void give(void* p, bool idle) {
+        if (!p) return;
+        std::lock_guard<std::mutex> lock(mu);
+        auto it = used.find(p);
+        if (it == used.end()) return;
+        const Block b = it->second;
+        used.erase(it);
+        if (b.bytes > POOL_BLOCK || !idle) {
+            (void)hipFree(b.p);
+            return;
+        }
+        shrink(POOL_BYTES - b.bytes);
+        try {
+            cached.push_back(b);
+            held += b.bytes;
+        } catch (...) {
+            (void)hipFree(b.p);
+        }
+    }
+
+    int device_of(void* p) {
+        std::lock_guard<std::mutex> lock(mu);
+        auto it = used.find(p);
+        return it == used.end() ? -1 : it->second.dev;
+    }
+
+    void shrink(size_t most) {                       // (with mu held)
+        size_t k = 0;
+        while (k < cached.size() && held > most) {
+            (void)hipFree(cached[k].p);
+            held -= cached[k++].bytes;
+        }
+        cached.erase(cached.begin(), cached.begin() + (std::ptrdiff_t)k);
+    }
+};
+
+// never destroyed: the runtime may be gone when static objects are
+DevPool& dev_pool() {
+    static DevPool* pool = new DevPool;
+    return *pool;
+}
+
+template <typename T>
+hipError_t dev_alloc(T** p, size_t bytes) {
+    void* v = nullptr;
+    const hipError_t e = dev_pool().take(&v, bytes);
+    *p = static_cast<T*>(v);
+    return e;
+}
+
+// Waits for a device; false where it cannot be waited for.
+bool dev_sync(int dev) {
+    int cur = 0;
+    if (hipGetDevice(&cur) != hipSuccess) return false;
+    if (cur != dev && hipSetDevice(dev) != hipSuccess) return false;
+    const bool ok = hipDeviceSynchronize() == hipSuccess;
+    if (cur != dev) (void)hipSetDevice(cur);
+    return ok;
+}
+
+void dev_give(void* p, bool idle) { dev_pool().give(p, idle); }
+
+void dev_free(void* p) {
+    if (!p) return;
+    const int dev = dev_pool().device_of(p);
+    if (dev >= 0) dev_give(p, dev_sync(dev));
+}
+
+}  // namespace
+
 // Device buffer freed on scope exit unless released.
 struct DevBuf {
     void* p = nullptr;
     DevBuf() = default;
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
-    ~DevBuf() { if (p) (void)hipFree(p); }
-    hipError_t alloc(size_t bytes) { return hipMalloc(&p, bytes ? bytes : 1); }
-    void* release() { void* r = p; p = nullptr; return r; }
+    ~DevBuf() { dev_free(p); }
+    hipError_t alloc(size_t bytes) { return dev_alloc(&p, bytes); }
     template <typename T> T* as() const { return static_cast<T*>(p); }
 };
 
@@ -309,10 +443,10 @@ static void choose_buckets(arb_field* f, ArbBuckets& B, bool table) {
 // first use.
 static int ensure_qrec(arb_field* f, int64_t n) {
     if (n > f->ws_qrec_n) {
-        if (f->ws_qrec) (void)hipFree(f->ws_qrec);
+        dev_free(f->ws_qrec);
         f->ws_qrec = nullptr;
         f->ws_qrec_n = 0;
-        HIPCHK(hipMalloc(&f->ws_qrec, (size_t)n * 16));
+        HIPCHK(dev_alloc(&f->ws_qrec, (size_t)n * 16));
         f->ws_qrec_n = n;
     }
     return ARB_OK;
@@ -321,10 +455,10 @@ static int ensure_qrec(arb_field* f, int64_t n) {
 // Room for `bytes` of packed output records, made on first use.
 static int ensure_records(arb_field* f, int64_t bytes) {
     if (bytes > f->ws_rec_bytes) {
-        if (f->ws_rec) (void)hipFree(f->ws_rec);
+        dev_free(f->ws_rec);
         f->ws_rec = nullptr;
         f->ws_rec_bytes = 0;
-        HIPCHK(hipMalloc(&f->ws_rec, (size_t)bytes));
+        HIPCHK(dev_alloc(&f->ws_rec, (size_t)bytes));
         f->ws_rec_bytes = bytes;
     }
     return ARB_OK;
@@ -430,7 +564,7 @@ int arb_field_create(const double* rows_dev, int64_t nrows, int32_t ncols, int64
     f->mode = mode;
     f->precision = precision;
     f->ninterp = interp_count(mode, &f->has_comps, &f->has_norm);
-    HIPCHK(hipMalloc(&f->flag, sizeof(int32_t) * 4));
+    HIPCHK(dev_alloc(&f->flag, sizeof(int32_t) * 4));
     HIPCHK(hipMemsetAsync(f->flag, 0, sizeof(int32_t) * 4, s));
 
     // 1. unique values per axis (and that coordinates are finite): one pass
@@ -532,7 +666,7 @@ int arb_field_create(const double* rows_dev, int64_t nrows, int32_t ncols, int64
     const int64_t seen_bytes = (g.nnodes + 7) / 8 * 8;
     HIPCHK(seen.alloc(seen_bytes));
     HIPCHK(hipMemsetAsync(seen.p, 0, seen_bytes, s));
-    HIPCHK(hipMalloc(&f->vals, sizeof(double) * g.nnodes * f->ninterp));
+    HIPCHK(dev_alloc(&f->vals, sizeof(double) * g.nnodes * f->ninterp));
     HIPCHK(arb_launch_rank_scatter(rows_dev, nrows, ld, axp, g, mode | f32_norm, ndim, f->vals,
                                    seen.as<unsigned char>(), s));
     HIPCHK(arb_launch_check_seen(seen.as<unsigned char>(), g.nnodes, f->flag, s));
@@ -547,7 +681,7 @@ int arb_field_create(const double* rows_dev, int64_t nrows, int32_t ncols, int64
     // the table itself is allocated by its first build (node-tile queries
     // never read it)
     f->table_bytes = (int64_t)((g.nc + 1) * f->ninterp * K * esz);
-    HIPCHK(hipMalloc(&f->sent, esz * f->ninterp * K));
+    HIPCHK(dev_alloc(&f->sent, esz * f->ninterp * K));
     HIPCHK(hipStreamSynchronize(s));
     guard.f = nullptr;
     *out = f;
@@ -615,8 +749,8 @@ int arb_field_set_boundary(arb_field* f, int32_t bc, void* stream) {
     HIPCHK(nv.alloc(sizeof(double) * gn.nnodes * f->ninterp));
     HIPCHK(arb_launch_pad_boundary(f->vals, go, nv.as<double>(), gn, f->ninterp, bc, s));
     HIPCHK(hipStreamSynchronize(s));
-    (void)hipFree(f->vals);
-    if (f->table) (void)hipFree(f->table);    // not built yet: allocated again by the build
+    dev_free(f->vals);
+    dev_free(f->table);    // not built yet: allocated again by the build
     f->vals = nv.as<double>();
     f->table = nullptr;
     nv.p = nullptr;
@@ -652,7 +786,7 @@ static int ensure_table_alloc(arb_field* f) {
     if (f->table) return ARB_OK;
     if (!f->otf && f->table_limit > 0 && f->table_bytes > f->table_limit) f->otf = 1;
     if (!f->otf) {
-        const hipError_t e = hipMalloc(&f->table, (size_t)f->table_bytes);
+        const hipError_t e = dev_alloc(&f->table, (size_t)f->table_bytes);
         if (e == hipErrorOutOfMemory) {
             (void)hipGetLastError();
             f->table = nullptr;
@@ -704,10 +838,10 @@ static int ensure_tiles(arb_field* f, hipStream_t s) {
     if (f->tiles_ok) return ARB_OK;
     const int64_t tb = arb_tiles_bytes(f->B, f->ninterp, nullptr);
     if (tb != f->tiles_bytes) {
-        if (f->tiles) (void)hipFree(f->tiles);
+        dev_free(f->tiles);
         f->tiles = nullptr;
         f->tiles_bytes = 0;
-        HIPCHK(hipMalloc(&f->tiles, (size_t)tb));
+        HIPCHK(dev_alloc(&f->tiles, (size_t)tb));
         f->tiles_bytes = tb;
     }
     HIPCHK(arb_launch_build_tiles(f->g, f->B, f->ninterp, f->vals, f->tiles, s));
@@ -758,10 +892,10 @@ static int64_t carve_sort_ws(unsigned char* base, int64_t n, int64_t nbt, bool q
 static int ensure_workspace(arb_field* f, int64_t n, int64_t nbt, SortWs* w) {
     const int64_t need = carve_sort_ws(nullptr, n, nbt, false, w);
     if (need > f->ws_bytes) {
-        if (f->ws) (void)hipFree(f->ws);
+        dev_free(f->ws);
         f->ws = nullptr;
         f->ws_bytes = 0;
-        HIPCHK(hipMalloc(&f->ws, (size_t)need));
+        HIPCHK(dev_alloc(&f->ws, (size_t)need));
         f->ws_bytes = need;
     }
     carve_sort_ws(static_cast<unsigned char*>(f->ws), n, nbt, false, w);
@@ -771,10 +905,10 @@ static int ensure_workspace(arb_field* f, int64_t n, int64_t nbt, SortWs* w) {
 // Bucket, rank and position per query (ARB_Q_GROUP_ATOMIC), made on first use.
 static int ensure_group(arb_field* f, int64_t n) {
     if (n > f->ws_group_n) {
-        if (f->ws_group) (void)hipFree(f->ws_group);
+        dev_free(f->ws_group);
         f->ws_group = nullptr;
         f->ws_group_n = 0;
-        HIPCHK(hipMalloc(&f->ws_group, sizeof(int32_t) * 3 * n));
+        HIPCHK(dev_alloc(&f->ws_group, sizeof(int32_t) * 3 * n));
         f->ws_group_n = n;
     }
     return ARB_OK;
@@ -1218,14 +1352,14 @@ int arb_query_backward(arb_field* f, const double* q_dev, int64_t n, int64_t ldq
     const int64_t nc = f->g.nc;
     if (dval_dev) {
         if (n > f->bw_n) {
-            if (f->bw_key) (void)hipFree(f->bw_key);
-            if (f->bw_perm) (void)hipFree(f->bw_perm);
-            if (f->bw_rec) (void)hipFree(f->bw_rec);
-            if (f->bw_k1) (void)hipFree(f->bw_k1);
-            if (f->bw_v1) (void)hipFree(f->bw_v1);
-            if (f->bw_hist) (void)hipFree(f->bw_hist);
-            if (f->bw_hscan) (void)hipFree(f->bw_hscan);
-            if (f->bw_part) (void)hipFree(f->bw_part);
+            dev_free(f->bw_key);
+            dev_free(f->bw_perm);
+            dev_free(f->bw_rec);
+            dev_free(f->bw_k1);
+            dev_free(f->bw_v1);
+            dev_free(f->bw_hist);
+            dev_free(f->bw_hscan);
+            dev_free(f->bw_part);
             f->bw_key = f->bw_perm = f->bw_v1 = f->bw_hist = f->bw_hscan = nullptr;
             f->bw_k1 = nullptr;
             f->bw_part = nullptr;
@@ -1233,21 +1367,21 @@ int arb_query_backward(arb_field* f, const double* q_dev, int64_t n, int64_t ldq
             f->bw_n = 0;
             const int64_t m = n ? n : 1;
             const int64_t hl = 256 * arb_rs_ntiles(m);
-            HIPCHK(hipMalloc(&f->bw_key, sizeof(int32_t) * m));
-            HIPCHK(hipMalloc(&f->bw_perm, sizeof(int32_t) * m));
-            HIPCHK(hipMalloc(&f->bw_k1, sizeof(uint32_t) * m));
-            HIPCHK(hipMalloc(&f->bw_v1, sizeof(int32_t) * m));
-            HIPCHK(hipMalloc(&f->bw_hist, sizeof(int32_t) * hl));
-            HIPCHK(hipMalloc(&f->bw_hscan, sizeof(int32_t) * (hl + 256)));
-            HIPCHK(hipMalloc(&f->bw_part, sizeof(double) * arb_bwd_part_elems(f->g, m)));
-            HIPCHK(hipMalloc(&f->bw_rec, sizeof(double) * arb_bwd_rec_elems(f->g) * m));
+            HIPCHK(dev_alloc(&f->bw_key, sizeof(int32_t) * m));
+            HIPCHK(dev_alloc(&f->bw_perm, sizeof(int32_t) * m));
+            HIPCHK(dev_alloc(&f->bw_k1, sizeof(uint32_t) * m));
+            HIPCHK(dev_alloc(&f->bw_v1, sizeof(int32_t) * m));
+            HIPCHK(dev_alloc(&f->bw_hist, sizeof(int32_t) * hl));
+            HIPCHK(dev_alloc(&f->bw_hscan, sizeof(int32_t) * (hl + 256)));
+            HIPCHK(dev_alloc(&f->bw_part, sizeof(double) * arb_bwd_part_elems(f->g, m)));
+            HIPCHK(dev_alloc(&f->bw_rec, sizeof(double) * arb_bwd_rec_elems(f->g) * m));
             f->bw_n = n;
         }
         if (!f->bw_bbar) {
             // the radix sort's first positions, then the cell bounds
-            HIPCHK(hipMalloc(&f->bw_count, sizeof(int32_t) * arb_rs_first_elems(nc)));
-            HIPCHK(hipMalloc(&f->bw_offs, sizeof(int32_t) * (nc + 1)));
-            HIPCHK(hipMalloc(&f->bw_bbar, sizeof(double) * arb_bwd_scratch(f->g)));
+            HIPCHK(dev_alloc(&f->bw_count, sizeof(int32_t) * arb_rs_first_elems(nc)));
+            HIPCHK(dev_alloc(&f->bw_offs, sizeof(int32_t) * (nc + 1)));
+            HIPCHK(dev_alloc(&f->bw_bbar, sizeof(double) * arb_bwd_scratch(f->g)));
         }
     }
     // The node adjoint groups the queries per cell in query-index order (so
@@ -1404,9 +1538,9 @@ int arb_batch_create(arb_field* const* fields, int32_t nfields, void* stream, ar
     HIPCHK(hipDeviceGetAttribute(&b->ncu, hipDeviceAttributeMultiprocessorCount, dev));
     const size_t dsz = arb_batch_field_desc_size();
     b->desc_host.assign(dsz * nfields, 0);
-    HIPCHK(hipMalloc(&b->desc_dev, dsz * nfields));
-    HIPCHK(hipMalloc(&b->counter, sizeof(unsigned int)));
-    HIPCHK(hipMalloc(&b->flag, sizeof(int32_t)));
+    HIPCHK(dev_alloc(&b->desc_dev, dsz * nfields));
+    HIPCHK(dev_alloc(&b->counter, sizeof(unsigned int)));
+    HIPCHK(dev_alloc(&b->flag, sizeof(int32_t)));
     HIPCHK(hipMemsetAsync(b->flag, 0, sizeof(int32_t), (hipStream_t)stream));
     HIPCHK(hipStreamSynchronize((hipStream_t)stream));
     for (arb_field* f : b->fields)
@@ -1498,9 +1632,9 @@ void arb_batch_destroy(arb_batch* b) {
     for (arb_field* f : b->fields)
         if (f) f->batches.erase(std::remove(f->batches.begin(), f->batches.end(), b),
                                 f->batches.end());
-    if (b->desc_dev) (void)hipFree(b->desc_dev);
-    if (b->counter) (void)hipFree(b->counter);
-    if (b->flag) (void)hipFree(b->flag);
+    dev_free(b->desc_dev);
+    dev_free(b->counter);
+    dev_free(b->flag);
     delete b;
 }
 
@@ -1512,7 +1646,7 @@ int arb_set_table_limit(arb_field* f, int64_t max_bytes) {
             return fail(ARB_EINVAL, "the loaded coefficient table (%lld bytes) exceeds the limit",
                         (long long)f->table_bytes);
         HIPCHK(hipDeviceSynchronize());     // no queued work may still read the table
-        (void)hipFree(f->table);
+        dev_free(f->table);
         f->table = nullptr;
         f->table_built = 0;
     }
@@ -1606,26 +1740,27 @@ void arb_field_destroy(arb_field* f) {
         for (auto& bf : b->fields)
             if (bf == f) bf = nullptr;
     }
-    if (f->vals) (void)hipFree(f->vals);
-    if (f->tiles) (void)hipFree(f->tiles);
-    if (f->table) (void)hipFree(f->table);
-    if (f->sent) (void)hipFree(f->sent);
-    if (f->flag) (void)hipFree(f->flag);
-    if (f->ws) (void)hipFree(f->ws);
-    if (f->ws_group) (void)hipFree(f->ws_group);
-    if (f->ws_rec) (void)hipFree(f->ws_rec);
-    if (f->ws_qrec) (void)hipFree(f->ws_qrec);
-    if (f->bw_key) (void)hipFree(f->bw_key);
-    if (f->bw_perm) (void)hipFree(f->bw_perm);
-    if (f->bw_k1) (void)hipFree(f->bw_k1);
-    if (f->bw_v1) (void)hipFree(f->bw_v1);
-    if (f->bw_hist) (void)hipFree(f->bw_hist);
-    if (f->bw_hscan) (void)hipFree(f->bw_hscan);
-    if (f->bw_part) (void)hipFree(f->bw_part);
-    if (f->bw_rec) (void)hipFree(f->bw_rec);
-    if (f->bw_count) (void)hipFree(f->bw_count);
-    if (f->bw_offs) (void)hipFree(f->bw_offs);
-    if (f->bw_bbar) (void)hipFree(f->bw_bbar);
+    const bool idle = dev_sync(f->device);          // the field's queued work is done
+    dev_give(f->vals, idle);
+    dev_give(f->tiles, idle);
+    dev_give(f->table, idle);
+    dev_give(f->sent, idle);
+    dev_give(f->flag, idle);
+    dev_give(f->ws, idle);
+    dev_give(f->ws_group, idle);
+    dev_give(f->ws_rec, idle);
+    dev_give(f->ws_qrec, idle);
+    dev_give(f->bw_key, idle);
+    dev_give(f->bw_perm, idle);
+    dev_give(f->bw_k1, idle);
+    dev_give(f->bw_v1, idle);
+    dev_give(f->bw_hist, idle);
+    dev_give(f->bw_hscan, idle);
+    dev_give(f->bw_part, idle);
+    dev_give(f->bw_rec, idle);
+    dev_give(f->bw_count, idle);
+    dev_give(f->bw_offs, idle);
+    dev_give(f->bw_bbar, idle);
     if (f->ev_ready)
         for (auto& e : f->ev) (void)hipEventDestroy(e);
     if (f->push_exec) (void)hipGraphExecDestroy(f->push_exec);
