@@ -325,6 +325,7 @@ struct arb_field {
     ArbBuckets B{};
     ArbBuckets BF{};
     int32_t user_block[ARB_MAXD] = {0, 0, 0, 0};
+    int32_t tableless = 0;         // a query has left the table out by its size
     int32_t eval_threads = 256;
     void* ws = nullptr;         // sort workspace (carve_sort_ws), one allocation
     int64_t ws_bytes = 0;
@@ -371,7 +372,8 @@ struct arb_field {
 // this trades 0.06 ms of evaluation (fewer workgroups per CU) for a 0.08 ms
 // sort pass.  The 3D on-the-fly kernel stores no coefficients: its largest
 // block, 4 x 4 x 4, forms the fewest passes per cell and has rows for every
-// wave (128^3 FP64 'both', 10^7 rows: 0.94 ms; 4 x 4 x 2 cells: 1.7 ms).
+// wave (128^3 FP64 'both', 10^7 rows: 0.94 ms; 4 x 4 x 2 cells: 1.7 ms).  The
+// 4D one has one block (arb_fused4.h).
 static int64_t bucket_count(const arb_field* f, const int* dims) {
     int64_t nb = 1;
     for (int a = 0; a < f->g.ndim; ++a) nb *= (f->g.npos[a] + dims[a] - 1) / dims[a];
@@ -389,7 +391,10 @@ static void choose_buckets(arb_field* f, ArbBuckets& B, bool table) {
                                      {2, 2, 1, 1}, {2, 1, 1, 1}, {1, 1, 1, 1}};
     const int max_cells = (48 * 1024) / (B.cellstride * 16);
     int dims[4] = {1, 1, 1, 1};
-    if (f->user_block[0] > 0) {
+    if (d == 4 && !table) {
+        static const int fused4[4] = {4, 4, 2, 1};
+        for (int a = 0; a < 4; ++a) dims[a] = fused4[a];
+    } else if (f->user_block[0] > 0) {
         for (int a = 0; a < d; ++a) dims[a] = f->user_block[a];
     } else {
         const int big_cells = (80 * 1024) / (B.cellstride * 16);
@@ -952,14 +957,7 @@ static int query_impl(arb_field* f, double* q_dev, int64_t n, int64_t ldq, void*
     ArbGeom gq = f->g;
     gq.red32 = red32 ? 1 : 0;
     bool sorted = (flags & (ARB_Q_SORTED | ARB_Q_SORTED_GLOBAL)) != 0;
-    // automatic choice: the bucketed path from about one query per four cells
-    // with node tiles (it stages ~128 bytes per cell), from one per two cells
-    // with the table (1 KB per cell in mixed 'both'); measured crossovers on
-    // the 128^3 field: 0.5 M and 1-2 M queries
-    if (!(flags & ARB_Q_DIRECT) && !sorted)
-        sorted = n >= 65536 && (node_path(f, flags) ? 4 * n : 2 * n) >= f->g.nc;
-    if (n > INT32_MAX - 1) sorted = false;
-    if (sorted && f->B.nbt == 0) choose_buckets(f, f->B, true);
+    const bool automatic = !(flags & ARB_Q_DIRECT) && !sorted;
     // 3D, bucketed: coefficients formed in the query kernel from node values,
     // no table, with the table's bits (not once a table has been loaded).  On
     // request, and by itself for FP64 fields of three or four interpolants
@@ -970,15 +968,40 @@ static int query_impl(arb_field* f, double* q_dev, int64_t n, int64_t ldq, void*
     // 0.044 / 0.042 for a table of 107 MB, which stays cached; one interpolant
     // gains nothing either (0.29 / 0.25 on 128^3 and 2 10^6 rows).  A block
     // chosen by the caller is the table kernel's.
+    // 4D likewise up to 2.5 rows per cell, with any number of interpolants
+    // (evaluation, ms, this kernel / the table's): one interpolant of 48^3 x 16
+    // nodes (2.4 GB of table), 2e6 rows 0.46 / 0.71, 6e5 rows 0.40 / 0.67, 2e6
+    // rows in a cloud 0.28 / 0.27; 40 x 37 x 30 x 12 nodes, 6.5 rows per cell:
+    // four interpolants 0.92 / 1.18, but in a cloud 0.76 / 0.45, and one
+    // interpolant 0.29 / 0.20.  FP32 tables are half the bytes: 0.45 / 0.30.
     constexpr int64_t kInfinityCache = (int64_t)256 << 20;
-    const bool by_size = f->precision == ARB_PREC_FP64 && f->ninterp >= 3 &&
-                         f->table_bytes > kInfinityCache && f->user_block[0] == 0 && !noalloc &&
-                         !(flags & ARB_Q_TABLE);
-    bool fused = false;
-    if (((flags & ARB_Q_FUSED) || by_size) && sorted && f->g.ndim == 3 && !f->table_loaded &&
-        !(flags & (ARB_Q_SORTED_GLOBAL | ARB_Q_GROUP_ATOMIC))) {
+    const int64_t nc = f->g.nc;
+    const bool no_table = f->precision == ARB_PREC_FP64 && f->table_bytes > kInfinityCache &&
+                          f->user_block[0] == 0 && !f->table_loaded &&
+                          !(flags & (ARB_Q_TABLE | ARB_Q_SORTED_GLOBAL | ARB_Q_GROUP_ATOMIC)) &&
+                          (!noalloc || (!f->table && f->tableless));
+    const bool by_size =
+        no_table && (f->g.ndim == 3 ? f->ninterp >= 3
+                                    : noalloc || 2 * n <= 5 * nc);
+    // automatic choice: the bucketed path from about one query per four cells
+    // with node tiles (it stages ~128 bytes per cell), from one per two cells
+    // with the table (1 KB per cell in mixed 'both'); measured crossovers on
+    // the 128^3 field: 0.5 M and 1-2 M queries
+    if (automatic) sorted = n >= 65536 && (node_path(f, flags) ? 4 * n : 2 * n) >= nc;
+    // an allocation-free call on a field that queries without a table
+    if (noalloc && by_size) sorted = true;
+    if (n > INT32_MAX - 1) sorted = false;
+    if (sorted && f->B.nbt == 0) choose_buckets(f, f->B, true);
+    const bool grouped = sorted && !f->table_loaded &&
+                         !(flags & (ARB_Q_SORTED_GLOBAL | ARB_Q_GROUP_ATOMIC));
+    bool fused = false, fused4 = false;
+    if (grouped && f->g.ndim == 3 && ((flags & ARB_Q_FUSED) || by_size)) {
         if (f->BF.nbt == 0) choose_buckets(f, f->BF, false);
         fused = arb_fused_ok(f->g, f->BF, f->ninterp);
+    }
+    if (grouped && f->g.ndim == 4 && ((flags & ARB_Q_FUSED) || by_size)) {
+        if (f->BF.nbt == 0) choose_buckets(f, f->BF, false);
+        fused4 = arb_fused4_ok(f->g, f->BF);
     }
     // node tiles (mixed 3D): the direct path, and the bucketed path unless
     // another grouping or the fused kernel is asked for; no table
@@ -986,12 +1009,11 @@ static int query_impl(arb_field* f, double* q_dev, int64_t n, int64_t ldq, void*
                  !(flags & (ARB_Q_SORTED_GLOBAL | ARB_Q_GROUP_ATOMIC));
     // a table path whose table does not fit: coefficients on the fly, in the
     // fused bucketed kernels (3D and 4D), whatever path was asked for
-    bool fused4 = false;
-    if (!fused && !nodes && !f->table && !noalloc) {
+    if (!fused && !fused4 && !nodes && !f->table && !noalloc) {
         const int rc0 = ensure_table_alloc(f);
         if (rc0 && !f->otf) return rc0;
     }
-    if (!fused && !nodes && f->otf) {
+    if (!fused && !fused4 && !nodes && f->otf) {
         if (red32)
             return fail(ARB_ENOMEM, "%s: the float32 reduction reads the coefficient table, which "
                         "does not fit", fn);
@@ -1003,7 +1025,7 @@ static int query_impl(arb_field* f, double* q_dev, int64_t n, int64_t ldq, void*
         if (f->g.ndim == 3)
             fused = arb_fused_ok(f->g, f->BF, f->ninterp);
         else
-            fused4 = arb_fused4_lds(f->g, f->BF) > 0;
+            fused4 = arb_fused4_ok(f->g, f->BF);
         if (!fused && !fused4)
             return fail(ARB_ENOMEM, "%s: the coefficient table does not fit and the bucket of "
                         "this field is too large to form its coefficients on the fly", fn);
@@ -1018,6 +1040,7 @@ static int query_impl(arb_field* f, double* q_dev, int64_t n, int64_t ldq, void*
             return fail(ARB_EINVAL, "%s: the field's coefficient table is not allocated; "
                         "prepare the field with arb_build_coeffs", fn);
     }
+    if ((fused || fused4) && by_size) f->tableless = 1;
     int rc = (fused || fused4 || nodes) ? ensure_sentinel(f, s) : arb_build_coeffs(f, stream);
     if (rc) return rc;
     if (nodes) {
@@ -1201,7 +1224,7 @@ static int query_impl(arb_field* f, double* q_dev, int64_t n, int64_t ldq, void*
         else if (fused4)
             HIPCHK(arb_launch_eval_fused4(f->g, BB, f->precision, out64, f->vals, f->ninterp,
                                           f->has_comps, f->has_norm, q_dev, n, ldq, o, offs,
-                                          perm, hot, f->eval_threads, s));
+                                          perm, hot, s));
         else
             HIPCHK(arb_launch_eval_bucket(f->g, f->B, f->precision, out64, f->table, f->ninterp,
                                           f->has_comps, f->has_norm, q_dev, n, ldq, o,

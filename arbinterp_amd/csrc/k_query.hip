@@ -5,7 +5,7 @@
 // gradients.  The reference builds ~40 N x 64 temporaries per call; here each
 // query is one lane.
 #include "arb_internal.h"
-#include "arb_sep4.h"
+#include "arb_fused4.h"
 
 namespace {
 
@@ -743,6 +743,28 @@ __device__ __forceinline__ void eval_row_lds(const ArbGeom& g, const ArbBuckets&
     eval_point<D, T, TC, TO>(a, has_comps, has_norm, loc, g, o, qi);
 }
 
+// The rows of chunk o, past the first chunk of their bucket.
+__device__ __forceinline__ bool chunk_rows(const int32_t* __restrict__ offs, int64_t nbt,
+                                           const int32_t* __restrict__ hot, int32_t chunk,
+                                           int64_t o, int64_t* b, int32_t* start, int32_t* end) {
+    if (hot[0] == 0) return false;
+    const int64_t p0 = o * (int64_t)chunk;
+    if (p0 >= offs[nbt]) return false;              // the rows outside the grid follow
+    int64_t lo = 0, hi = nbt;                       // offs[lo] <= p0 < offs[hi]
+    while (hi - lo > 1) {
+        const int64_t mid = (lo + hi) >> 1;
+        if (offs[mid] <= p0) lo = mid;
+        else hi = mid;
+    }
+    const int64_t s0 = (int64_t)offs[lo] + chunk, e0 = offs[lo + 1];
+    const int64_t s1 = p0 > s0 ? p0 : s0;
+    const int64_t e1 = p0 + chunk < e0 ? p0 + chunk : e0;
+    *b = lo;
+    *start = (int32_t)s1;
+    *end = (int32_t)e1;
+    return s1 < e1;
+}
+
 // Rows of the bucketed evaluation taken by this workgroup (uniform over it).
 // Workgroup w < nbt takes the first `chunk` rows of bucket w.  Workgroup
 // nbt + o takes, among the sorted positions [o chunk, (o + 1) chunk), the
@@ -763,22 +785,7 @@ __device__ __forceinline__ bool bucket_rows(const int32_t* __restrict__ offs, in
         *end = e0 - s0 > chunk ? s0 + chunk : e0;
         return s0 < e0;
     }
-    if (hot[0] == 0) return false;
-    const int64_t p0 = (w - nbt) * (int64_t)chunk;
-    if (p0 >= offs[nbt]) return false;              // the rows outside the grid follow
-    int64_t lo = 0, hi = nbt;                       // offs[lo] <= p0 < offs[hi]
-    while (hi - lo > 1) {
-        const int64_t mid = (lo + hi) >> 1;
-        if (offs[mid] <= p0) lo = mid;
-        else hi = mid;
-    }
-    const int64_t s0 = (int64_t)offs[lo] + chunk, e0 = offs[lo + 1];
-    const int64_t s1 = p0 > s0 ? p0 : s0;
-    const int64_t e1 = p0 + chunk < e0 ? p0 + chunk : e0;
-    *b = lo;
-    *start = (int32_t)s1;
-    *end = (int32_t)e1;
-    return s1 < e1;
+    return chunk_rows(offs, nbt, hot, chunk, w - nbt, b, start, end);
 }
 
 // One workgroup per bucket: stage the block's coefficients in LDS, then
@@ -980,8 +987,9 @@ k_eval_fused3(ArbGeom g, ArbBuckets B, const double* __restrict__ vals,
         int lc[R], rank[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            if (!local_cell<BX, BY, BZ>(qp[r], g, c0, loc[r], &lc[r])) {
-                // beside the block: an aliased index (a coordinate at IntMax)
+            if (!local_cell<BX, BY, BZ>(qp[r], g, c0, loc[r], &lc[r]) && qi[r] >= 0) {
+                // beside the block: an aliased index (a coordinate at IntMax;
+                // about 500 instructions, not for lanes without a row)
                 int64_t ia[3];
                 bool oob;
                 const int64_t flat = arb_reduce_axes<3>(qp[r], g, loc[r], ia, &oob);
@@ -1170,148 +1178,222 @@ k_eval_fused3(ArbGeom g, ArbBuckets B, const double* __restrict__ vals,
 }
 
 // ---------------------------------------------------------------------------
-// 4D without the coefficient table (the table does not fit, or a table size
-// limit is set): one workgroup per bucket forms its cells' coefficients in
-// LDS with the arithmetic of the 4D table build (arb_sep4.h: per power of t
-// the t-combined 3D node tile through the separable passes, then the
-// row-shift correction P . c with c_k = G(k-1) - G(k), row 85 zero; and NaN
-// for every coefficient of a cell whose stencil holds a non-finite value),
-// so the results are bitwise those of the table, and evaluates the bucket's
-// queries as the staged kernel does.  Dynamic LDS: the coefficient block
-// (ncell * cellstride * 16 bytes), then doubles: the block's 4D node tile,
-// one t-combined 3D tile, the pass buffers, the corner differences G and
-// the per-cell c.
+// 4D without the coefficient table: one workgroup per bucket of 4 x 4 x 2 x 1
+// cells evaluates its rows from node values, four lanes to a row
+// (arb_fused4.h), with the operations of the table build and of the table
+// kernels (arb_val4, arb_valgrad4) in their order, so the results are bitwise
+// those of the table.  The lane of power et of t evaluates that slice; along t
+// every lane of the quad finishes one derivative (et 0..2: x, y, z; 3: t and
+// the value) and writes its part of the row.
+//
+// 48^3 x 16 nodes, FP64, one interpolant, 2e6 rows (1.7 per cell): 0.46 ms,
+// against 0.71 ms for the staged table kernel, which reads 2.4 GB (and whose
+// table takes 0.53 ms to build); 6e5 rows 0.40 against 0.67 ms.  About 0.2 ms
+// of it is VALU issue and 0.18 ms LDS; the rest is what two waves per SIMD
+// leave of the barriers between the passes.  Measured without gain: one layer
+// per workgroup (0.75 ms: the chain bounds -> row index -> position and the
+// node loads), rows put in cell order first (0.49 ms: LDS conflicts fall from
+// three ways to none, two barriers a batch more), two rows of a cell per quad
+// (0.61 ms: 256 registers and spills).
 // ---------------------------------------------------------------------------
-template <int BX, int BY, int BZ, int BT>
-struct Fused4Shape {
-    static constexpr int NX = BX + 3, NY = BY + 3, NZ = BZ + 3, NTT = BT + 3;
-    static constexpr int NT4 = NX * NY * NZ * NTT;                 // node tile
-    static constexpr int NT3 = NX * NY * NZ;                       // t-combined tile
-    static constexpr int GX = BX + 1, GY = BY + 1, GZ = BZ + 1, GT = BT + 1;
-    static constexpr int NG = GX * GY * GZ * GT;                   // corner differences
-    static constexpr int NC = BX * BY * BZ * BT;
-    static constexpr int DOUBLES = NT4 + NT3 + (NY * NZ * BX * 4) + (NZ * BY * BX * 16) + NG + NC * 16;
-};
-
-template <typename T, typename TO, int BX, int BY, int BZ, int BT>
-__global__ void __launch_bounds__(256)
+template <typename T, typename TO>
+__global__ void __launch_bounds__(arbf4::TH)
 k_eval_fused4(ArbGeom g, ArbBuckets B, const double* __restrict__ vals, int32_t ninterp,
               int32_t has_comps, int32_t has_norm, const double* __restrict__ q, int64_t n,
               int64_t ldq, ArbOut o, const int32_t* __restrict__ offs,
-              const int32_t* __restrict__ perm, const int32_t* __restrict__ hot) {
-    using S = Fused4Shape<BX, BY, BZ, BT>;
-    extern __shared__ uint4 smem[];
-    __shared__ unsigned char cbad[S::NC];           // cells with a non-finite stencil
-    int64_t b;
-    int32_t start, end;
-    if (!bucket_rows(offs, B.nbt, hot, ARB_EVAL_CHUNK, &b, &start, &end)) return;
-    int64_t c0[4];
-    bucket_origin<4>(b, B, c0);
-    double* nodes = reinterpret_cast<double*>(smem + B.ncell * B.cellstride);
-    double* t3 = nodes + S::NT4;
-    double* t1 = t3 + S::NT3;
-    double* t2 = t1 + S::NY * S::NZ * BX * 4;
-    double* gcorn = t2 + S::NZ * BY * BX * 16;
-    double* cc = gcorn + S::NG;
-    T* cf = reinterpret_cast<T*>(smem);
-    const int cstr = B.cellstride * (16 / (int)sizeof(T));   // elements per LDS cell
-    // this thread's first query, loaded before the coefficient work
-    int32_t s = start + threadIdx.x;
-    int64_t qi = -1;
-    double qp[4];
-    if (s < end) {
-        const int64_t pi = perm[s];
-        qi = (pi >= 0 && pi < n) ? pi : -1;         // always in range: perm holds row indices
-        const int64_t qq = qi >= 0 ? qi : 0;
-#pragma unroll
-        for (int a = 0; a < 4; ++a) qp[a] = q[qq * ldq + a];
+              const int32_t* __restrict__ perm, const int32_t* __restrict__ hot, int32_t ncol,
+              int32_t nseg, int32_t seg) {
+    using namespace arbf4;
+    __shared__ __align__(16) Smem S;
+    // workgroup w < ncol nseg: layers [l0, l1) of the block w % ncol, the
+    // first chunk of rows of each; then the chunks of rows past it
+    const int tid = threadIdx.x, et = tid & 3;
+    const int32_t w = (int32_t)blockIdx.x;
+    int64_t col;
+    int32_t l0, l1;
+    if (w < ncol * nseg) {
+        col = w % ncol;
+        l0 = w / ncol * seg;
+        l1 = l0 + seg < (int32_t)B.nb[3] ? l0 + seg : (int32_t)B.nb[3];
+        int2 r = make_int2(0, 0);
+        if (tid < l1 - l0) {
+            const int64_t b = col + (int64_t)ncol * (l0 + tid);
+            r = make_int2(offs[b], offs[b + 1]);
+            if (r.y - r.x > ARB_EVAL_CHUNK) r.y = r.x + ARB_EVAL_CHUNK;
+        }
+        if (tid < SEG) S.rows[tid] = r;
+        if (!__syncthreads_or(r.x < r.y)) return;
+    } else {
+        int64_t b;
+        int32_t start, end;
+        if (!chunk_rows(offs, B.nbt, hot, ARB_EVAL_CHUNK, w - ncol * nseg, &b, &start, &end)) return;
+        col = b % ncol;
+        l0 = (int32_t)(b / ncol);
+        l1 = l0 + 1;
+        if (tid == 0) S.rows[0] = make_int2(start, end);
+        __syncthreads();
     }
+    // layers without rows at either end are left out
+    const int32_t base = l0;
+    while (S.rows[l0 - base].x >= S.rows[l0 - base].y) ++l0;
+    while (S.rows[l1 - 1 - base].x >= S.rows[l1 - 1 - base].y) --l1;
+    int64_t c0[4];
+    bucket_origin<4>(col, B, c0);
+    // the quad's row: its index (-1 for none), position, local cell and
+    // coordinates
+    int32_t qi;
+    int lc;
+    double qp, loc;                                 // of the lane's axis
+    const Axis axis = lane_axis(g, et);
+    // perm at the quad's row of a layer (loaded only, so that nothing waits
+    // for it yet), and that row's index once it is needed
+    auto load_index = [&](int32_t layer, int32_t more) -> int32_t {
+        const int2 r = S.rows[(layer < l1 ? layer : l0) - base];
+        const int32_t s = r.x + (tid >> 2) + more;
+        return perm[s < r.y ? s : 0];
+    };
+    auto index = [&](int32_t layer, int32_t more, int32_t i) -> int32_t {
+        const int2 r = S.rows[layer - base];
+        return r.x + (tid >> 2) + more < r.y && i < n ? i : -1;     // perm holds row indices
+    };
+    auto next = [&](int32_t& t, int32_t& s) {
+        const int2 r = S.rows[t - base];
+        s += ROWS;
+        if (s >= r.y - r.x) {
+            ++t;
+            s = 0;
+        }
+    };
+    auto fetch = [&](int32_t i) -> double { return q[(i >= 0 ? (int64_t)i : 0) * ldq + et]; };
+    const int b0 = (int)c0[0], b1 = (int)c0[1], b2 = (int)c0[2];
+    auto place = [&](int32_t t) {
+        // a row of another bucket cannot happen (same reduction as k_keys)
+        if (!place_row(qp, axis, g, b0, b1, b2, t, &loc, &lc)) qi = -1;
+        if (qi < 0) lc = 0;
+    };
+    TO* const rec = reinterpret_cast<TO*>(o.comps);
+    Column C;
+    column_origin(g, c0, C);
+    C.next = 0.0;
     for (int k = 0; k < ninterp; ++k) {
         const double* F = vals + (int64_t)k * g.nnodes;
-        __syncthreads();                            // the previous interpolant is done
-        // node tile, x fastest then y, z, t; nodes past the grid read 0 (only
-        // cells outside the grid use them)
-        int nonfinite = 0;
-        for (int e = threadIdx.x; e < S::NT4; e += blockDim.x) {
-            const int x = e % S::NX, y = (e / S::NX) % S::NY, z = (e / (S::NX * S::NY)) % S::NZ;
-            const int t = e / (S::NX * S::NY * S::NZ);
-            const int64_t nx = c0[0] + x, ny = c0[1] + y, nz = c0[2] + z, nt = c0[3] + t;
-            double v = 0.0;
-            if (nx < g.n[0] && ny < g.n[1] && nz < g.n[2] && nt < g.n[3])
-                v = F[nx + g.nstride[1] * ny + g.nstride[2] * nz + g.nstride[3] * nt];
-            nodes[e] = v;
-            nonfinite |= !isfinite(v);
-        }
-        const bool anybad = __syncthreads_or(nonfinite) != 0;
-        auto N4 = [&](int x, int y, int z, int t) {
-            return nodes[((t * S::NZ + z) * S::NY + y) * S::NX + x];
-        };
-        if (anybad) {
-            for (int c = threadIdx.x; c < S::NC; c += blockDim.x) {
-                const int cx = c % BX, cy = (c / BX) % BY, cz = (c / (BX * BY)) % BZ;
-                const int ct = c / (BX * BY * BZ);
-                bool bad = false;
-                for (int t = 0; t < 4; ++t)
-                    for (int z = 0; z < 4; ++z)
-                        for (int y = 0; y < 4; ++y)
-                            for (int x = 0; x < 4; ++x)
-                                bad |= !isfinite(N4(cx + x, cy + y, cz + z, ct + t));
-                cbad[c] = bad ? 1 : 0;
+        // steps: the batches of 64 rows of a layer, then the next layer's
+        int32_t in = load_index(l0, 0);             // of the next step's row
+        if (k > 0) __syncthreads();                 // nodes read by the previous one's passes
+        column_start(F, g, l0, C, S);
+        qi = index(l0, 0, in);
+        qp = fetch(qi);
+        int32_t t = l0, s = 0, t1 = l0, s1 = 0;
+        next(t1, s1);
+        in = load_index(t1, s1);
+        bool half = false, anybad = false;
+        while (t < l1) {
+            const int32_t count = S.rows[t - base].y - S.rows[t - base].x;
+            if (s == 0) anybad = __syncthreads_or(C.nf != 0) != 0;
+            place(t);
+            // loads of the next step: its rows, the indices of the rows after
+            // them, and the next layer's last plane
+            int32_t qn = -1, t2 = t1, s2 = s1;
+            double qpn = 0.0;
+            if (s == 0 && t + 1 < l1) C.next = column_load(F, g, C, t + 4);
+            if (t1 < l1) {
+                qn = index(t1, s1, in);
+                qpn = fetch(qn);
+                next(t2, s2);
+                in = load_index(t2, s2);
             }
-        }
-        // xyzt central differences at the cells' corner nodes (tile node + 1),
-        // in the table build's order of terms
-        for (int i = threadIdx.x; i < S::NG; i += blockDim.x) {
-            const int gx = i % S::GX, gy = (i / S::GX) % S::GY, gz = (i / (S::GX * S::GY)) % S::GZ;
-            const int gt = i / (S::GX * S::GY * S::GZ);
-            gcorn[i] = arbs4::corner_diff<S::NX, S::NX * S::NY, S::NX * S::NY * S::NZ>(
-                nodes + (((gt + 1) * S::NZ + gz + 1) * S::NY + gy + 1) * S::NX + gx + 1);
-        }
-        __syncthreads();
-        // c_k = G(corner k-1) - G(corner k) per cell
-        for (int i = threadIdx.x; i < S::NC * 16; i += blockDim.x) {
-            const int kk = i & 15, c = i >> 4;
-            const int cx = c % BX, cy = (c / BX) % BY, cz = (c / (BX * BY)) % BZ;
-            const int ct = c / (BX * BY * BZ);
-            auto G = [&](int cn) {
-                const int gx = cx + (cn & 1), gy = cy + ((cn >> 1) & 1);
-                const int gz = cz + ((cn >> 2) & 1), gt = ct + ((cn >> 3) & 1);
-                return gcorn[((gt * S::GZ + gz) * S::GY + gy) * S::GX + gx];
-            };
-            cc[c * 16 + kk] = (kk ? G(kk - 1) : 0.0) - G(kk);
-        }
-        for (int ct = 0; ct < BT; ++ct) {
-            for (int et = 0; et < 4; ++et) {
-                // t-combined 3D node tile for power et of cell row ct
-                for (int i = threadIdx.x; i < S::NT3; i += blockDim.x) {
-                    const int x = i % S::NX, y = (i / S::NX) % S::NY, z = i / (S::NX * S::NY);
-                    double c[4];
-                    arbs3::cub4(N4(x, y, z, ct), N4(x, y, z, ct + 1), N4(x, y, z, ct + 2),
-                                N4(x, y, z, ct + 3), c);
-                    t3[i] = c[et];
+            // they are waited for before this step's stores are issued: loads
+            // and stores count in one counter, and a wait behind the stores
+            // would be for them too
+            auto arrived = [&]() { asm volatile("" ::"v"(qpn), "v"(in), "v"(C.next)); };
+            if (count > 0) {
+                if (s == 0) {
+                    passes_t(t, C, half, anybad, S);
+                    __syncthreads();
+                    passes_xy(t, S);
+                    __syncthreads();
                 }
-                __syncthreads();
-                arbs3::sep3_passes4<BX, BY, BZ, false>(
-                    t3, t1, t2, [&](int cx, int cy, int cz, int exy, const double* c0) {
-                        const int c = cx + BX * (cy + BY * (cz + BZ * ct));
-                        double a[4] = {c0[0], c0[1], c0[2], c0[3]};
-                        arbs4::shift_rows(cc + c * 16, exy & 3, exy >> 2, et, a);
-                        const bool bad = anybad && cbad[c];
-                        T* o = cf + c * cstr + k * 256 + exy + 64 * et;
-#pragma unroll
-                        for (int ez = 0; ez < 4; ++ez) o[16 * ez] = bad ? (T)NAN : (T)a[ez];
-                    });
+                if (s + ((tid & ~63) >> 2) < count) {       // rows in this wave
+                    T x[4];
+                    quad_all((T)loc, x);
+                const bool bad = anybad && S.bad[lc];
+                if (has_norm && k == ninterp - 1) {
+                    T qv[4], qd[4], qu[4];
+    #pragma unroll
+                    for (int ey = 3; ey >= 0; --ey) {
+                        T al[4][4];
+                        coef<T>(S, lc, et, ey, al);
+    #pragma unroll
+                        for (int ez = 0; ez < 4; ++ez) {
+                            T p, pu;
+                            h4d<T>(al[0][ez], al[1][ez], al[2][ez], al[3][ez], x[0], p, pu);
+                            stream_h4d<T>(ey, p, x[1], qv[ez], qd[ez]);
+                            stream_h4<T>(ey, pu, x[1], qu[ez]);
+                        }
+                    }
+                    T r, rw;
+                    h4d<T>(qv[0], qv[1], qv[2], qv[3], x[2], r, rw);
+                    const T ru = h4<T>(qu[0], qu[1], qu[2], qu[3], x[2]);
+                    const T rv = h4<T>(qd[0], qd[1], qd[2], qd[3], x[2]);
+                    T au[4], av[4], aw[4], ar[4], f[4];
+                    quad_all(ru, au);
+                    quad_all(rv, av);
+                    quad_all(rw, aw);
+                    quad_all(r, ar);
+    #pragma unroll
+                    for (int l = 0; l < 4; ++l) f[l] = pick(et, au[l], av[l], aw[l], ar[l]);
+                    T p, dp;
+                    h4d<T>(f[0], f[1], f[2], f[3], x[3], p, dp);
+                    if (bad) p = dp = (T)NAN;       // a non-finite stencil: NaN throughout
+                    const TO gr = (TO)((et == 3 ? dp : p) / (T)axis.h);
+                    arrived();
+                    if (qi >= 0) {
+                        const int at = has_comps ? 3 : 0;
+                        if (o.packed) {
+                            TO* w = rec + (int64_t)qi * o.packed;
+                            w[at + 1 + et] = gr;
+                            if (et == 3) w[at] = (TO)p;
+                            if (at + 5 + et < o.packed) w[at + 5 + et] = (TO)0;
+                        } else {
+                            put<TO>(o.grads, (int64_t)qi * 4 + et, gr);
+                            if (et == 3) put<TO>(o.norms, qi, (TO)p);
+                        }
+                    }
+                } else {
+                    T qv[4];
+    #pragma unroll
+                    for (int ey = 3; ey >= 0; --ey) {
+                        T al[4][4];
+                        coef<T>(S, lc, et, ey, al);
+    #pragma unroll
+                        for (int ez = 0; ez < 4; ++ez)
+                            stream_h4<T>(ey, h4<T>(al[0][ez], al[1][ez], al[2][ez], al[3][ez], x[0]),
+                                         x[1], qv[ez]);
+                    }
+                    T ar[4];
+                    quad_all(h4<T>(qv[0], qv[1], qv[2], qv[3], x[2]), ar);
+                    const TO val = (TO)(bad ? (T)NAN : h4<T>(ar[0], ar[1], ar[2], ar[3], x[3]));
+                    arrived();
+                    if (qi >= 0 && et == 0) {
+                        if (o.packed) {
+                            rec[(int64_t)qi * o.packed + k] = val;
+                            if (k == 2 && !has_norm) rec[(int64_t)qi * o.packed + 3] = (TO)0;
+                        } else {
+                            put<TO>(o.comps, (int64_t)qi * 3 + k, val);
+                        }
+                    }
+                }
+                }
             }
+            if (t1 > t) half = count > 0;
+            if (t1 > t && t1 < l1) column_step(t1, C, S);
+            qi = qn;
+            qp = qpn;
+            t = t1;
+            s = s1;
+            t1 = t2;
+            s1 = s2;
         }
-    }
-    __syncthreads();
-    if (qi >= 0) eval_row_lds<4, T, T, TO>(g, B, smem, has_comps, has_norm, o, b, qi, qp);
-    for (s += blockDim.x; s < end; s += blockDim.x) {
-        const int64_t pi = perm[s];
-        if (pi < 0 || pi >= n) continue;            // unreachable: perm holds row indices
-#pragma unroll
-        for (int a = 0; a < 4; ++a) qp[a] = q[pi * ldq + a];
-        eval_row_lds<4, T, T, TO>(g, B, smem, has_comps, has_norm, o, b, pi, qp);
     }
 }
 
@@ -2230,54 +2312,38 @@ hipError_t arb_launch_eval_fused(const ArbGeom& g, const ArbBuckets& B, int32_t 
     return hipErrorInvalidValue;
 }
 
-// Cell blocks of the 4D fused kernel (the 4D bucket ladder).
-#define ARB_FUSED4_SHAPES(X)                                                                  \
-    X(4, 4, 2, 2) X(4, 2, 2, 2) X(2, 2, 2, 2) X(2, 2, 2, 1) X(2, 2, 1, 1) X(2, 1, 1, 1)      \
-    X(1, 1, 1, 1)
-
-// LDS bytes of k_eval_fused4 for the bucket geometry B (0 when it does not
-// apply: 4D, an instantiated block shape, the local cell index laid out as
-// the kernel writes it, within 160 KiB with its static LDS).
-size_t arb_fused4_lds(const ArbGeom& g, const ArbBuckets& B) {
-    if (g.ndim != 4) return 0;
-    const int bx = B.b[0], by = B.b[1], bz = B.b[2], bt = B.b[3];
-    size_t dbl = 0;
-#define ARB_F4_IS(X, Y, Z, T)                                                                 \
-    if (bx == X && by == Y && bz == Z && bt == T) dbl = Fused4Shape<X, Y, Z, T>::DOUBLES;
-    ARB_FUSED4_SHAPES(ARB_F4_IS)
-#undef ARB_F4_IS
-    if (dbl == 0) return 0;
-    if (B.lsh[0] != 0 || (1 << B.lsh[1]) != bx || (1 << B.lsh[2]) != bx * by ||
-        (1 << B.lsh[3]) != bx * by * bz)
-        return 0;
-    const size_t lds = (size_t)B.ncell * B.cellstride * 16 + sizeof(double) * dbl;
-    return lds + 256 <= 160 * 1024 ? lds : 0;
+// Whether k_eval_fused4 takes the bucket geometry B: 4D, its block, the local
+// cell index cx + bx (cy + by cz).
+bool arb_fused4_ok(const ArbGeom& g, const ArbBuckets& B) {
+    return g.ndim == 4 && B.b[0] == arbf4::BX && B.b[1] == arbf4::BY && B.b[2] == arbf4::BZ &&
+           B.b[3] == 1 && B.lsh[0] == 0 && (1 << B.lsh[1]) == arbf4::BX &&
+           (1 << B.lsh[2]) == arbf4::BX * arbf4::BY;
 }
 
 hipError_t arb_launch_eval_fused4(const ArbGeom& g, const ArbBuckets& B, int32_t prec,
                                   int32_t out_f64, const double* vals, int32_t ninterp,
                                   int32_t has_comps, int32_t has_norm, const double* q, int64_t n,
                                   int64_t ldq, const ArbOut& o, const int32_t* offs,
-                                  const int32_t* perm, const int32_t* hot, int32_t block_threads,
-                                  hipStream_t s) {
-    (void)block_threads;
-    const size_t lds = arb_fused4_lds(g, B);
-    if (lds == 0) return hipErrorInvalidValue;
-    dim3 grid(eval_grid(B, n)), block(arbs3::SEP_THREADS);
-#define L_FUSED4(T, TO, X, Y, Z, TT)                                                          \
-    hipLaunchKernelGGL((k_eval_fused4<T, TO, X, Y, Z, TT>), grid, block, lds, s, g, B, vals,  \
-                       ninterp, has_comps, has_norm, q, n, ldq, o, offs, perm, hot)
-#define ARB_FUSED4_CASE(X, Y, Z, TT)                                                          \
-    if (B.b[0] == X && B.b[1] == Y && B.b[2] == Z && B.b[3] == TT) {                          \
-        if (prec == ARB_PREC_FP64) L_FUSED4(double, double, X, Y, Z, TT);                     \
-        else if (out_f64) L_FUSED4(float, double, X, Y, Z, TT);                               \
-        else L_FUSED4(float, float, X, Y, Z, TT);                                             \
-        return hipGetLastError();                                                             \
-    }
-    ARB_FUSED4_SHAPES(ARB_FUSED4_CASE)
-#undef ARB_FUSED4_CASE
+                                  const int32_t* perm, const int32_t* hot, hipStream_t s) {
+    if (!arb_fused4_ok(g, B)) return hipErrorInvalidValue;
+    // layers of t per workgroup: as many as leave about ten workgroups for
+    // each of the chip's 512 places (48^3 x 16 nodes: 7 of 13)
+    const int64_t ncol = B.nb[0] * B.nb[1] * B.nb[2], nt = B.nb[3];
+    int64_t nseg = (5120 + ncol - 1) / ncol;
+    if (nseg * arbf4::SEG < nt) nseg = (nt + arbf4::SEG - 1) / arbf4::SEG;
+    if (nseg > nt) nseg = nt;
+    const int64_t seg = (nt + nseg - 1) / nseg;
+    nseg = (nt + seg - 1) / seg;
+    dim3 grid((unsigned)(ncol * nseg + (n + ARB_EVAL_CHUNK - 1) / ARB_EVAL_CHUNK)), block(arbf4::TH);
+#define L_FUSED4(T, TO)                                                                       \
+    hipLaunchKernelGGL((k_eval_fused4<T, TO>), grid, block, 0, s, g, B, vals, ninterp,         \
+                       has_comps, has_norm, q, n, ldq, o, offs, perm, hot, (int32_t)ncol,      \
+                       (int32_t)nseg, (int32_t)seg)
+    if (prec == ARB_PREC_FP64) L_FUSED4(double, double);
+    else if (out_f64) L_FUSED4(float, double);
+    else L_FUSED4(float, float);
 #undef L_FUSED4
-    return hipErrorInvalidValue;
+    return hipGetLastError();
 }
 
 // Cell blocks the node-tile kernels are instantiated for.// Cell blocks the node-tile kernels are instantiated for.

@@ -90,11 +90,12 @@ extern "C" {
                                arb_field_info.packed_width elements into
                                comps_dev: [comps(3)] [value, grad(d)], zero
                                padded; norms_dev/grads_dev are not used        */
-#define ARB_Q_FUSED  1024   /* 3D bucketed path: form each block's
+#define ARB_Q_FUSED  1024   /* bucketed path: form each block's
                                coefficients in the query kernel from node
                                values instead of staging them from the table.
                                No table is built or read; the results are
-                               bitwise those of the table-reading paths      */
+                               bitwise those of the table-reading paths (the
+                               default for large FP64 fields)                */
 #define ARB_Q_SORT_CELL 512  /* bucketed path: order queries by bucket, then by
                                cell inside the bucket (default: bucket only)    */
 #define ARB_Q_TABLE  2048   /* read each cell's coefficients from the table
@@ -103,7 +104,7 @@ extern "C" {
                                paths: each query is evaluated from its 4x4x4
                                node values, no table is built or read; results
                                agree with the table path to FP32 rounding,
-                               not bitwise)                                   */
+                               not bitwise), or ARB_Q_FUSED by the field's size */
 
 #define ARB_Q_REDUCE_F32 4096 /* the field and the positions were float32 in the
                                caller (the values here are their exact FP64
@@ -221,7 +222,8 @@ int arb_query(arb_field* f, double* q_dev, int64_t n, int64_t ldq,
  *   - the field must already hold its coefficient table (table paths:
  *     arb_build_coeffs) or node tiles (mixed 3D: one arb_query with the same
  *     flags, n may be 0); they are rebuilt in place after
- *     arb_field_set_values.  Otherwise ARB_EINVAL;
+ *     arb_field_set_values.  A large FP64 field that an arb_query has answered
+ *     without a table needs neither.  Otherwise ARB_EINVAL;
  *   - n <= ARB_NOALLOC_MAX_ROWS, and the workspace of n rows over the field's
  *     buckets must fit the array (about 16 bytes per row, 32 on the mixed 3D
  *     node-tile path, plus 8 per bucket), else ARB_EINVAL with the sizes in
