@@ -919,6 +919,48 @@ static int ensure_group(arb_field* f, int64_t n) {
     return ARB_OK;
 }
 
+// Whether n rows are worth grouping (the bucketed path) when the caller leaves
+// the choice open; both paths give the same bits.  The direct kernel's time is
+// the rows' (a cell's coefficients each), the bucketed path's that of the sort
+// (about 80 us), of the cells, and little per row, so it pays from a number of
+// rows on and from a density on.  Measured at the lines, us direct / bucketed,
+// uniform rows on few cells (3D 184e3, 4D 41e3) and on many (3D 2e6, 4D 1.2e6
+// for one interpolant, else 3.1e5):
+//   3D FP64   1 interpolant   2e6 rows 182/188;   3e6 rows (1.5 per cell) 368/380
+//             3               4e5 113/113;        1e6 (0.5) 397/409
+//             4               3.2e5 130/138;      4.9e5 (0.25) 600/568
+//   3D mixed  1               1e6 108/123;        1e6 (0.5) 166/184
+//             3               2.5e5 83/80;        5e5 (0.25) 200/162
+//             4               2.5e5 84/94;        5e5 (0.25) 218/197
+//   4D FP64   1               2.5e5 94/92;        6e5 (0.5) 330/480, in a cloud 213/210
+//             3               1.5e5 164/151;      2.5e5 (0.8) 339/490
+//             4               1e5 192/175;        2.5e5 (0.8) 486/645
+//   4D mixed  1               8e5 136/119;        1e6 (0.84) 250/360, in a cloud 160/169
+//             3, 4            1e5 103/100, 128/126;  2.5e5 (0.8) 278/440, 344/480
+// In 4D uniform rows would cross at 0.85 to 1.7 rows per cell, rows in a cloud
+// (which touch fewer cells) from 0.5: the line lies where neither loses to the
+// former one.  That was 65536 rows and one per two cells, per four with node
+// tiles: 2.5e5 rows of the small 3D grid and one interpolant took 92 us for
+// 30, 1e6 rows of the large one 289 for 126.  A field that queries without its
+// table (by_size) and has none is taken from there on: the direct kernel would
+// build it first.
+static bool bucketed_pays(arb_field* f, int64_t n, int32_t flags, bool by_size) {
+    const int64_t nc = f->g.nc;
+    const bool mixed = f->precision == ARB_PREC_MIXED, one = f->ninterp == 1;
+    if (f->g.ndim == 4) {
+        const int64_t least = one ? (mixed ? 800000 : 262144)
+                                  : (mixed || f->ninterp == 4 ? 98304 : 163840);
+        return n >= least && (!one ? 4 * n >= 3 * nc : mixed ? 8 * n >= 7 * nc : 2 * n >= nc);
+    }
+    if (by_size && !f->table_built && n >= 65536 && 2 * n >= nc) return true;
+    if (mixed && node_path(f, flags))
+        return n >= (one ? 1000000 : f->ninterp == 3 ? 245760 : 286720) &&
+               (one ? 2 : 4) * n >= nc;
+    if (mixed) return n >= 65536 && 2 * n >= nc;
+    return n >= (one ? 2097152 : f->ninterp == 3 ? 393216 : 327680) &&
+           (one ? 2 * n >= 3 * nc : (by_size && f->ninterp == 4 ? 4 : 2) * n >= nc);
+}
+
 // arb_query and arb_query_noalloc.  With noalloc the call allocates nothing:
 // the table or node tiles must already be allocated (they are rebuilt in
 // place when the node values changed), the bucketed path takes its sort
@@ -983,11 +1025,7 @@ static int query_impl(arb_field* f, double* q_dev, int64_t n, int64_t ldq, void*
     const bool by_size =
         no_table && (f->g.ndim == 3 ? f->ninterp >= 3
                                     : noalloc || 2 * n <= 5 * nc);
-    // automatic choice: the bucketed path from about one query per four cells
-    // with node tiles (it stages ~128 bytes per cell), from one per two cells
-    // with the table (1 KB per cell in mixed 'both'); measured crossovers on
-    // the 128^3 field: 0.5 M and 1-2 M queries
-    if (automatic) sorted = n >= 65536 && (node_path(f, flags) ? 4 * n : 2 * n) >= nc;
+    if (automatic) sorted = bucketed_pays(f, n, flags, by_size);
     // an allocation-free call on a field that queries without a table
     if (noalloc && by_size) sorted = true;
     if (n > INT32_MAX - 1) sorted = false;
