@@ -211,18 +211,27 @@ constexpr int BN = BB + 3;                         // node tile edge
 constexpr int BCELLS = BB * BB * BB;
 constexpr int BTILE = BN * BN * BN;
 
-// A cell holding more than BWD_CHUNK queries is summed in pieces: the
+// A cell holding more than C queries is summed in pieces: the
 // queries at sorted positions [o C, (o + 1) C) of such a cell (C =
-// BWD_CHUNK, o C inside the cell) are summed by a chunk kernel into
+// BWD_CHUNK_OF, o C inside the cell) are summed by a chunk kernel into
 // part[o], in index order, and the cell's own sum takes the queries before
 // its first multiple of C in index order, then part[o] for each of its
 // chunks in order: a fixed order, so the result still repeats bit for bit,
 // and a cell of many queries (particles clustered in a few cells) is
 // spread over many threads instead of four.
-constexpr int32_t BWD_CHUNK = 1024;
+//
+// A thread group adds a cell's queries one after another, about 2 us each (the
+// chain perm -> record), and the partial sums about 1 us each, so the chunk
+// balances the two; 1024 in both dimensions left clouds of particles waiting
+// for a few cells.  Forward + backward of 1e6 queries in a cloud (ms, chunk
+// 1024 / now): 3D mixed 25^3 nodes 3.9 / 1.4, 50^3 4.0 / 1.5, 96^3 0.87 / 0.88
+// (with chunks of 128: 1.0, 1.0 and 1.14, its cells of some 150 queries then
+// taking two kernels); 4D FP64 22 x 24 x 22 x 10 nodes 5.0 / 1.2.
+template <int D>
+constexpr int32_t BWD_CHUNK_OF = D == 3 ? 256 : 128;
 
 // The chunk starting at sorted position o C, if it belongs to a cell of
-// more than BWD_CHUNK queries: [s0, s1) and that cell; q, ldq: the query
+// more than BWD_CHUNK_OF queries: [s0, s1) and that cell; q, ldq: the query
 // positions (the cell of the query at o C, by the same reduction as the
 // keys).
 template <int D>
@@ -230,7 +239,7 @@ __device__ __forceinline__ bool bwd_chunk(const ArbGeom& g, const double* __rest
                                           int64_t ldq, const int32_t* __restrict__ offs,
                                           const int32_t* __restrict__ perm, int64_t o,
                                           int32_t* s0, int32_t* s1) {
-    const int64_t p0 = o * BWD_CHUNK;
+    const int64_t p0 = o * BWD_CHUNK_OF<D>;
     if (p0 >= offs[g.nc]) return false;              // the rows outside the box follow
     const int64_t i = perm[p0];
     double loc[D];
@@ -238,9 +247,9 @@ __device__ __forceinline__ bool bwd_chunk(const ArbGeom& g, const double* __rest
     const int64_t c = arb_reduce<D>(q + i * ldq, g, loc, &oob);
     if (c < 0 || c >= g.nc) return false;            // cannot happen: p0 is a cell's row
     const int32_t e = offs[c + 1];
-    if (e - offs[c] <= BWD_CHUNK) return false;      // summed whole by the cell kernel
+    if (e - offs[c] <= BWD_CHUNK_OF<D>) return false;      // summed whole by the cell kernel
     *s0 = (int32_t)p0;
-    *s1 = p0 + BWD_CHUNK < e ? (int32_t)(p0 + BWD_CHUNK) : e;
+    *s1 = p0 + BWD_CHUNK_OF<D> < e ? (int32_t)(p0 + BWD_CHUNK_OF<D>) : e;
     return true;
 }
 
@@ -342,15 +351,15 @@ k_bwd_block3(ArbGeom g, const double* __restrict__ rec, const int32_t* __restric
         if (x < g.npos[0] && y < g.npos[1] && z < g.npos[2]) {
             const int64_t c = x + g.npos[0] * (y + g.npos[1] * z);
             const int32_t s0 = offs[c], s1 = offs[c + 1];
-            if (s1 - s0 <= BWD_CHUNK) {
+            if (s1 - s0 <= BWD_CHUNK_OF<3>) {
                 abar_rows3<1>(rec, rperm, s0, s1, gq, acc);
             } else {
                 // the queries before the cell's first chunk, then its chunks
-                const int64_t ofirst = ((int64_t)s0 + BWD_CHUNK - 1) / BWD_CHUNK;
-                const int32_t h1 = ofirst * BWD_CHUNK < s1 ? (int32_t)(ofirst * BWD_CHUNK) : s1;
+                const int64_t ofirst = ((int64_t)s0 + BWD_CHUNK_OF<3> - 1) / BWD_CHUNK_OF<3>;
+                const int32_t h1 = ofirst * BWD_CHUNK_OF<3> < s1 ? (int32_t)(ofirst * BWD_CHUNK_OF<3>) : s1;
                 abar_rows3<1>(rec, rperm, s0, h1, gq, acc);
                 // then the chunks' sums, in chunk order
-                for (int64_t o = ofirst; o * BWD_CHUNK < s1; ++o) {
+                for (int64_t o = ofirst; o * BWD_CHUNK_OF<3> < s1; ++o) {
 #pragma unroll
                     for (int p = 0; p < 4; ++p)
 #pragma unroll
@@ -560,7 +569,7 @@ __device__ __forceinline__ void sums4_rows(const double* __restrict__ rec, int32
     for (int32_t s = s0; s < s1; ++s) sums4_row(load_rec4(rec, s), gq, S);
 }
 
-// Chunk sums (cells of more than BWD_CHUNK queries): eight threads per
+// Chunk sums (cells of more than BWD_CHUNK_OF queries): eight threads per
 // chunk, part[o][sum][gq].
 __global__ void __launch_bounds__(256)
 k_bwd_chunk4(ArbGeom g, const double* __restrict__ q, int64_t ldq, const double* __restrict__ rec,
@@ -625,14 +634,14 @@ k_bwd_block4(ArbGeom g, const double* __restrict__ rec, const int32_t* __restric
         }
         if (idle == 0) {
             S.cb[0] = S.cb[1] = S.a85 = 0.0;
-            if (s1 - s0 <= BWD_CHUNK) {
+            if (s1 - s0 <= BWD_CHUNK_OF<4>) {
                 sums4_rows(rec, s0, s1, gq, S);
             } else {
                 // the queries before the cell's first chunk, then its chunks
-                const int64_t ofirst = ((int64_t)s0 + BWD_CHUNK - 1) / BWD_CHUNK;
-                const int32_t h1 = ofirst * BWD_CHUNK < s1 ? (int32_t)(ofirst * BWD_CHUNK) : s1;
+                const int64_t ofirst = ((int64_t)s0 + BWD_CHUNK_OF<4> - 1) / BWD_CHUNK_OF<4>;
+                const int32_t h1 = ofirst * BWD_CHUNK_OF<4> < s1 ? (int32_t)(ofirst * BWD_CHUNK_OF<4>) : s1;
                 sums4_rows(rec, s0, h1, gq, S);
-                for (int64_t o = ofirst; o * BWD_CHUNK < s1; ++o) {
+                for (int64_t o = ofirst; o * BWD_CHUNK_OF<4> < s1; ++o) {
                     const double* p = part + o * (8 * SUMS4) + gq;
 #pragma unroll
                     for (int i = 0; i < 32; ++i) S.ring[i >> 3][(i >> 2) & 1][i & 3] += p[8 * i];
@@ -835,8 +844,12 @@ int64_t arb_bwd_scratch(const ArbGeom& g) {
     return nb[0] * nb[1] * nb[2] * g.n[3] * TILE4;
 }
 
+static int64_t chunk_rows(const ArbGeom& g) {
+    return g.ndim == 3 ? BWD_CHUNK_OF<3> : BWD_CHUNK_OF<4>;
+}
+
 int64_t arb_bwd_part_elems(const ArbGeom& g, int64_t n) {
-    const int64_t nchunk = (n + BWD_CHUNK - 1) / BWD_CHUNK;
+    const int64_t nchunk = (n + chunk_rows(g) - 1) / chunk_rows(g);
     return (nchunk ? nchunk : 1) * (g.ndim == 3 ? 64 : 8 * SUMS4);
 }
 
@@ -844,7 +857,7 @@ hipError_t arb_launch_bwd_cells(const ArbGeom& g, const double* q, int64_t ldq, 
                                 int32_t rec_grouped, const int32_t* offs, const int32_t* perm,
                                 int64_t n, double* part, double* bbar, hipStream_t s) {
     const int32_t* rperm = rec_grouped ? nullptr : perm;
-    const int64_t nchunk = (n + BWD_CHUNK - 1) / BWD_CHUNK;
+    const int64_t nchunk = (n + chunk_rows(g) - 1) / chunk_rows(g);
     int64_t nb[3];
     if (g.ndim == 3) {
         if (nchunk > 0)
