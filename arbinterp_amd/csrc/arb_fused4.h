@@ -273,30 +273,40 @@ __device__ __forceinline__ Axis lane_axis(const ArbGeom& g, int et) {
 
 // Local coordinate (of the lane's axis) and local cell of the quad's row in
 // the block of cells at (c0, c1, c2) and layer t; x: the lane's coordinate.
-// False for a row that is not in it.  A coordinate at IntMax gives a cell
-// index one past its axis, which the flat index carries into the next axis.
-__device__ __forceinline__ bool place_row(double x, const Axis& A, const ArbGeom& g, int c0, int c1,
-                                          int c2, int t, double* loc, int* lc) {
-    const double a = x - A.lo;
+// False for a row that is not in it.  row: whether the quad has one.  One
+// without takes IntMin, not x, which then is another row's and may lie
+// anywhere: nothing below may run on it.
+//
+// A row of the block is inside the box and its flat index below nc < 2^32.
+// Its index along an axis can still reach past the axis: a coordinate at
+// IntMax, or any beyond the cells that an axis whose first spacing is its
+// smallest counts.  Only then the flat index is decoded (bucket_of, in 32
+// bits), three divisions however far past it lies.
+__device__ __forceinline__ bool place_row(bool row, double x, const Axis& A, const ArbGeom& g,
+                                          int c0, int c1, int c2, int t, double* loc, int* lc) {
+    const double a = row ? x - A.lo : 0.0;
     double iu = a * A.rh;                           // arb_div_h
     iu = fma(fma(-iu, A.h, a), A.rh, iu);
     iu = fma(fma(-iu, A.h, a), A.rh, iu);
     if (A.rh == 0.0) iu = a / A.h;
     const double fl = floor(iu);
     *loc = iu - fl;
-    int i[4];
-    quad_all((int)fl, i);
-    if (i[0] >= (int)g.npos[0] || i[1] >= (int)g.npos[1] || i[2] >= (int)g.npos[2]) {
-#pragma unroll
-        for (int b = 0; b < 3; ++b)
-            while (i[b] >= (int)g.npos[b]) {
-                i[b] -= (int)g.npos[b];
-                ++i[b + 1];
-            }
+    int q[4];
+    quad_all((int)(uint32_t)fl, q);
+    const uint32_t n0 = (uint32_t)g.npos[0], n1 = (uint32_t)g.npos[1], n2 = (uint32_t)g.npos[2];
+    uint32_t i[4] = {(uint32_t)q[0], (uint32_t)q[1], (uint32_t)q[2], (uint32_t)q[3]};
+    if (i[0] >= n0 || i[1] >= n1 || i[2] >= n2) {
+        uint32_t rem = i[0] + n0 * (i[1] + n1 * (i[2] + n2 * i[3]));
+        i[0] = rem % n0;
+        rem /= n0;
+        i[1] = rem % n1;
+        rem /= n1;
+        i[2] = rem % n2;
+        i[3] = rem / n2;
     }
-    const int l0 = i[0] - c0, l1 = i[1] - c1, l2 = i[2] - c2;
-    *lc = l0 + BX * (l1 + BY * l2);
-    return (unsigned)l0 < BX && (unsigned)l1 < BY && (unsigned)l2 < BZ && i[3] == t;
+    const uint32_t l0 = i[0] - (uint32_t)c0, l1 = i[1] - (uint32_t)c1, l2 = i[2] - (uint32_t)c2;
+    *lc = (int)(l0 + BX * (l1 + BY * l2));
+    return l0 < (uint32_t)BX && l1 < (uint32_t)BY && l2 < (uint32_t)BZ && i[3] == (uint32_t)t;
 }
 
 }  // namespace arbf4

@@ -1268,7 +1268,7 @@ k_eval_fused4(ArbGeom g, ArbBuckets B, const double* __restrict__ vals, int32_t 
     const int b0 = (int)c0[0], b1 = (int)c0[1], b2 = (int)c0[2];
     auto place = [&](int32_t t) {
         // a row of another bucket cannot happen (same reduction as k_keys)
-        if (!place_row(qp, axis, g, b0, b1, b2, t, &loc, &lc)) qi = -1;
+        if (!place_row(qi >= 0, qp, axis, g, b0, b1, b2, t, &loc, &lc)) qi = -1;
         if (qi < 0) lc = 0;
     };
     TO* const rec = reinterpret_cast<TO*>(o.comps);
