@@ -299,12 +299,13 @@ hipError_t arb_launch_rk4(const ArbGeom& g, int32_t prec, const void* table, int
                           hipStream_t s) {
     if (n <= 0 || nsteps <= 0) return hipSuccess;
     dim3 grid(grid1(n, 256)), block(256);
-    // accel3_fast: cells and their flat indices (one past the last cell per
-    // axis included) in 32 bits, and magnitudes that keep div_h's residuals
-    // away from under- and overflow
+    // accel3_fast: flat cell indices in 32 bits, and magnitudes that keep
+    // div_h's residuals away from under- and overflow.  A position's index
+    // along an axis is at most (hi - lo) / h there (one for rounding): npos on
+    // an even axis, any number on one whose first spacing is its smallest
     PushGeom pg{};
     bool fast = true;
-    double cells = 1.0;
+    double top = 0.0, cells = 1.0;
     for (int d = 0; d < 3; ++d) {
         pg.lo[d] = g.lo[d];
         pg.hi[d] = g.hi[d];
@@ -312,12 +313,13 @@ hipError_t arb_launch_rk4(const ArbGeom& g, int32_t prec, const void* table, int
         pg.rh[d] = 1.0 / g.h[d];
         pg.rhg[d] = prec == ARB_PREC_FP64 ? pg.rh[d] : 1.0 / (double)(float)g.h[d];
         pg.np[d] = (int32_t)g.npos[d];
-        cells *= (double)g.npos[d] + 1.0;
+        top += ((g.hi[d] - g.lo[d]) / g.h[d] + 1.0) * cells;
+        cells *= (double)g.npos[d];
         const double e = 0x1p300;
         fast &= g.h[d] > 1.0 / e && g.h[d] < e && fabs(g.lo[d]) < e && fabs(g.hi[d]) < e;
         if (prec != ARB_PREC_FP64) fast &= g.h[d] > 0x1p-100 && g.h[d] < 0x1p100;
     }
-    fast &= cells < 2147483647.0;
+    fast &= top < 2147483647.0 && cells < 2147483647.0;
     pg.nc = (int32_t)g.nc;
 #define L_RK4(T, F)                                                                             \
     hipLaunchKernelGGL((k_rk4<T, T, F>), grid, block, 0, s, g, pg, (const T*)table, ninterp, kn, \
