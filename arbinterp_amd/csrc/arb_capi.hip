@@ -38,14 +38,15 @@ static int fail(int code, const char* fmt, ...) {
     } while (0)
 
 // ---------------------------------------------------------------------------
-// Device memory.  Blocks of up to POOL_BLOCK bytes come back to a pool of at
-// most POOL_BYTES for the whole process (the oldest leave first, and all of
-// them when an allocation fails), so a program that makes one field after
-// another (a field per time step) does not pay for mapping and unmapping its
-// node values and workspaces each time: 112 x 96 x 88 nodes and 10^6 queries,
-// hipFree alone took 1.3 of 1.9 ms.  Larger blocks (tables) are freed at once.
-// A block enters the pool when its device is idle (as hipFree waits for it to
-// be), so whatever thread or stream takes it next, nothing still uses it.
+// Device memory.  A destroyed field's blocks of up to POOL_BLOCK bytes go to a
+// pool of at most POOL_BYTES for the whole process (the oldest leave first,
+// and all of them when an allocation fails), so a program that makes one field
+// after another (a field per time step) does not pay for mapping and unmapping
+// its node values and workspaces each time: 112 x 96 x 88 nodes and 10^6
+// queries, hipFree alone took 1.3 of 1.9 ms.  Larger blocks (tables), and what
+// a living field gives up, are freed at once.  A block enters the pool when
+// nothing uses it any more (as hipFree waits for that), so whatever thread or
+// stream takes it next may write it.
 // ---------------------------------------------------------------------------
 namespace {
 
@@ -100,31 +101,24 @@ struct DevPool {
         return hipSuccess;
     }
 
-    // idle: the block's device has been waited for (else it is freed, which waits)
-    void give(void* p, bool idle) {
-        if (!p) return;
+    // idle: what used the block has been waited for (else it is freed, which
+    // waits)
+    hipError_t give(void* p, bool idle) {
+        if (!p) return hipSuccess;
         std::lock_guard<std::mutex> lock(mu);
         auto it = used.find(p);
-        if (it == used.end()) return;
+        if (it == used.end()) return hipErrorInvalidValue;
         const Block b = it->second;
         used.erase(it);
-        if (b.bytes > POOL_BLOCK || !idle) {
-            (void)hipFree(b.p);
-            return;
-        }
+        if (b.bytes > POOL_BLOCK || !idle) return hipFree(b.p);
         shrink(POOL_BYTES - b.bytes);
         try {
             cached.push_back(b);
             held += b.bytes;
         } catch (...) {
-            (void)hipFree(b.p);
+            return hipFree(b.p);
         }
-    }
-
-    int device_of(void* p) {
-        std::lock_guard<std::mutex> lock(mu);
-        auto it = used.find(p);
-        return it == used.end() ? -1 : it->second.dev;
+        return hipSuccess;
     }
 
     void shrink(size_t most) {                       // (with mu held)
@@ -151,33 +145,20 @@ hipError_t dev_alloc(T** p, size_t bytes) {
     return e;
 }
 
-// Waits for a device; false where it cannot be waited for.
-bool dev_sync(int dev) {
-    int cur = 0;
-    if (hipGetDevice(&cur) != hipSuccess) return false;
-    if (cur != dev && hipSetDevice(dev) != hipSuccess) return false;
-    const bool ok = hipDeviceSynchronize() == hipSuccess;
-    if (cur != dev) (void)hipSetDevice(cur);
-    return ok;
-}
+void dev_give(void* p, bool idle) { (void)dev_pool().give(p, idle); }
 
-void dev_give(void* p, bool idle) { dev_pool().give(p, idle); }
-
-void dev_free(void* p) {
-    if (!p) return;
-    const int dev = dev_pool().device_of(p);
-    if (dev >= 0) dev_give(p, dev_sync(dev));
-}
+hipError_t dev_free(void* p) { return dev_pool().give(p, false); }
 
 }  // namespace
 
-// Device buffer freed on scope exit unless released.
+// Device buffer of work on one stream, given back on scope exit unless released.
 struct DevBuf {
     void* p = nullptr;
-    DevBuf() = default;
+    hipStream_t s;
+    explicit DevBuf(hipStream_t stream) : s(stream) {}
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
-    ~DevBuf() { dev_free(p); }
+    ~DevBuf() { if (p) dev_give(p, hipStreamSynchronize(s) == hipSuccess); }
     hipError_t alloc(size_t bytes) { return dev_alloc(&p, bytes); }
     template <typename T> T* as() const { return static_cast<T*>(p); }
 };
@@ -448,7 +429,7 @@ static void choose_buckets(arb_field* f, ArbBuckets& B, bool table) {
 // first use.
 static int ensure_qrec(arb_field* f, int64_t n) {
     if (n > f->ws_qrec_n) {
-        dev_free(f->ws_qrec);
+        (void)dev_free(f->ws_qrec);
         f->ws_qrec = nullptr;
         f->ws_qrec_n = 0;
         HIPCHK(dev_alloc(&f->ws_qrec, (size_t)n * 16));
@@ -460,7 +441,7 @@ static int ensure_qrec(arb_field* f, int64_t n) {
 // Room for `bytes` of packed output records, made on first use.
 static int ensure_records(arb_field* f, int64_t bytes) {
     if (bytes > f->ws_rec_bytes) {
-        dev_free(f->ws_rec);
+        (void)dev_free(f->ws_rec);
         f->ws_rec = nullptr;
         f->ws_rec_bytes = 0;
         HIPCHK(dev_alloc(&f->ws_rec, (size_t)bytes));
@@ -578,7 +559,7 @@ int arb_field_create(const double* rows_dev, int64_t nrows, int32_t ncols, int64
     // values.  An axis of more than AXES_MAX takes hash sets sized for any
     // rows, an axis at a time.
     std::vector<std::vector<double>> axes(ndim);
-    DevBuf sets;
+    DevBuf sets(s);
     HIPCHK(sets.alloc(arb_axes_bytes(ndim)));
     const AxesLayout L = arb_axes_layout(sets.p, ndim);
     HIPCHK(hipMemsetAsync(L.hash, 0xFF, L.hash_bytes, s));
@@ -604,7 +585,7 @@ int arb_field_create(const double* rows_dev, int64_t nrows, int32_t ncols, int64
     } else {
         int64_t cap = 1024;
         while (cap < 2 * nrows) cap <<= 1;
-        DevBuf tab, uniq, cnt;
+        DevBuf tab(s), uniq(s), cnt(s);
         HIPCHK(tab.alloc(sizeof(unsigned long long) * cap));
         HIPCHK(uniq.alloc(sizeof(double) * cap));
         HIPCHK(cnt.alloc(sizeof(unsigned int)));
@@ -660,7 +641,7 @@ int arb_field_create(const double* rows_dev, int64_t nrows, int32_t ncols, int64
 
     // 2. rank rows, scatter values into canonical order, check that every node
     // was written (with as many rows as nodes, then each exactly once)
-    DevBuf axbuf, seen;
+    DevBuf axbuf(s), seen(s);
     std::vector<double> axall;
     const double* axp[ARB_MAXD] = {nullptr, nullptr, nullptr, nullptr};
     for (int a = 0; a < ndim; ++a) axall.insert(axall.end(), axes[a].begin(), axes[a].end());
@@ -750,12 +731,12 @@ int arb_field_set_boundary(arb_field* f, int32_t bc, void* stream) {
     const int K = 1 << (2 * go.ndim);
     const size_t esz = f->precision == ARB_PREC_FP64 ? sizeof(double) : sizeof(float);
     const int64_t tbytes = (int64_t)((gn.nc + 1) * f->ninterp * K * esz);
-    DevBuf nv;
+    DevBuf nv(s);
     HIPCHK(nv.alloc(sizeof(double) * gn.nnodes * f->ninterp));
     HIPCHK(arb_launch_pad_boundary(f->vals, go, nv.as<double>(), gn, f->ninterp, bc, s));
     HIPCHK(hipStreamSynchronize(s));
-    dev_free(f->vals);
-    dev_free(f->table);    // not built yet: allocated again by the build
+    (void)dev_free(f->vals);
+    (void)dev_free(f->table);    // not built yet: allocated again by the build
     f->vals = nv.as<double>();
     f->table = nullptr;
     nv.p = nullptr;
@@ -843,7 +824,7 @@ static int ensure_tiles(arb_field* f, hipStream_t s) {
     if (f->tiles_ok) return ARB_OK;
     const int64_t tb = arb_tiles_bytes(f->B, f->ninterp, nullptr);
     if (tb != f->tiles_bytes) {
-        dev_free(f->tiles);
+        (void)dev_free(f->tiles);
         f->tiles = nullptr;
         f->tiles_bytes = 0;
         HIPCHK(dev_alloc(&f->tiles, (size_t)tb));
@@ -897,7 +878,7 @@ static int64_t carve_sort_ws(unsigned char* base, int64_t n, int64_t nbt, bool q
 static int ensure_workspace(arb_field* f, int64_t n, int64_t nbt, SortWs* w) {
     const int64_t need = carve_sort_ws(nullptr, n, nbt, false, w);
     if (need > f->ws_bytes) {
-        dev_free(f->ws);
+        (void)dev_free(f->ws);
         f->ws = nullptr;
         f->ws_bytes = 0;
         HIPCHK(dev_alloc(&f->ws, (size_t)need));
@@ -910,7 +891,7 @@ static int ensure_workspace(arb_field* f, int64_t n, int64_t nbt, SortWs* w) {
 // Bucket, rank and position per query (ARB_Q_GROUP_ATOMIC), made on first use.
 static int ensure_group(arb_field* f, int64_t n) {
     if (n > f->ws_group_n) {
-        dev_free(f->ws_group);
+        (void)dev_free(f->ws_group);
         f->ws_group = nullptr;
         f->ws_group_n = 0;
         HIPCHK(dev_alloc(&f->ws_group, sizeof(int32_t) * 3 * n));
@@ -1413,14 +1394,14 @@ int arb_query_backward(arb_field* f, const double* q_dev, int64_t n, int64_t ldq
     const int64_t nc = f->g.nc;
     if (dval_dev) {
         if (n > f->bw_n) {
-            dev_free(f->bw_key);
-            dev_free(f->bw_perm);
-            dev_free(f->bw_rec);
-            dev_free(f->bw_k1);
-            dev_free(f->bw_v1);
-            dev_free(f->bw_hist);
-            dev_free(f->bw_hscan);
-            dev_free(f->bw_part);
+            (void)dev_free(f->bw_key);
+            (void)dev_free(f->bw_perm);
+            (void)dev_free(f->bw_rec);
+            (void)dev_free(f->bw_k1);
+            (void)dev_free(f->bw_v1);
+            (void)dev_free(f->bw_hist);
+            (void)dev_free(f->bw_hscan);
+            (void)dev_free(f->bw_part);
             f->bw_key = f->bw_perm = f->bw_v1 = f->bw_hist = f->bw_hscan = nullptr;
             f->bw_k1 = nullptr;
             f->bw_part = nullptr;
@@ -1693,9 +1674,9 @@ void arb_batch_destroy(arb_batch* b) {
     for (arb_field* f : b->fields)
         if (f) f->batches.erase(std::remove(f->batches.begin(), f->batches.end(), b),
                                 f->batches.end());
-    dev_free(b->desc_dev);
-    dev_free(b->counter);
-    dev_free(b->flag);
+    (void)dev_free(b->desc_dev);
+    (void)dev_free(b->counter);
+    (void)dev_free(b->flag);
     delete b;
 }
 
@@ -1707,7 +1688,7 @@ int arb_set_table_limit(arb_field* f, int64_t max_bytes) {
             return fail(ARB_EINVAL, "the loaded coefficient table (%lld bytes) exceeds the limit",
                         (long long)f->table_bytes);
         HIPCHK(hipDeviceSynchronize());     // no queued work may still read the table
-        dev_free(f->table);
+        (void)dev_free(f->table);
         f->table = nullptr;
         f->table_built = 0;
     }
@@ -1801,12 +1782,18 @@ void arb_field_destroy(arb_field* f) {
         for (auto& bf : b->fields)
             if (bf == f) bf = nullptr;
     }
-    const bool idle = dev_sync(f->device);          // the field's queued work is done
+    // the field's queued work, on whatever streams: waited for by freeing its
+    // status word (hipFree waits for the device; hipDeviceSynchronize would
+    // end a stream capture in progress, also a relaxed one)
+    int dev = f->device;
+    bool idle = hipGetDevice(&dev) == hipSuccess &&
+                (dev == f->device || hipSetDevice(f->device) == hipSuccess);
+    idle &= dev_free(f->flag) == hipSuccess;
+    if (dev != f->device) (void)hipSetDevice(dev);
     dev_give(f->vals, idle);
     dev_give(f->tiles, idle);
     dev_give(f->table, idle);
     dev_give(f->sent, idle);
-    dev_give(f->flag, idle);
     dev_give(f->ws, idle);
     dev_give(f->ws_group, idle);
     dev_give(f->ws_rec, idle);
