@@ -942,11 +942,19 @@ static bool bucketed_pays(arb_field* f, int64_t n, int32_t flags, bool by_size) 
            (one ? 2 * n >= 3 * nc : (by_size && f->ninterp == 4 ? 4 : 2) * n >= nc);
 }
 
+// Rows from which an allocation-free call without a table groups them.  Row by
+// row / grouped, us: 1 row 10/37, 1024 rows 11/59, 8192 58/114, 16384 112/116,
+// 32768 220/116 ('both', 90 x 66 x 41 nodes; the direct kernel with a table: 9,
+// 17 and, 16384 rows, 19); 16384 rows of 128^3 'both' 112/299, of one 4D
+// interpolant 102/111 (22 x 21 x 20 x 27 nodes) and 106/250 (48^3 x 16).
+constexpr int64_t kCellRows = 16384;
+
 // arb_query and arb_query_noalloc.  With noalloc the call allocates nothing:
 // the table or node tiles must already be allocated (they are rebuilt in
-// place when the node values changed), the bucketed path takes its sort
-// workspace from `scratch` and writes the output arrays directly (no packed
-// record workspace), and flags that need other workspaces are refused.
+// place when the node values changed) or an arb_query have been answered
+// without them, the bucketed path takes its sort workspace from `scratch` and
+// writes the output arrays directly (no packed record workspace), and flags
+// that need other workspaces are refused.
 static int query_impl(arb_field* f, double* q_dev, int64_t n, int64_t ldq, void* comps_dev,
                       void* norms_dev, void* grads_dev, int64_t* cells_dev, int32_t flags,
                       void* stream, bool noalloc) {
@@ -999,26 +1007,37 @@ static int query_impl(arb_field* f, double* q_dev, int64_t n, int64_t ldq, void*
     // interpolant 0.29 / 0.20.  FP32 tables are half the bytes: 0.45 / 0.30.
     constexpr int64_t kInfinityCache = (int64_t)256 << 20;
     const int64_t nc = f->g.nc;
-    const bool no_table = f->precision == ARB_PREC_FP64 && f->table_bytes > kInfinityCache &&
-                          f->user_block[0] == 0 && !f->table_loaded &&
-                          !(flags & (ARB_Q_TABLE | ARB_Q_SORTED_GLOBAL | ARB_Q_GROUP_ATOMIC)) &&
-                          (!noalloc || (!f->table && f->tableless));
     const bool by_size =
-        no_table && (f->g.ndim == 3 ? f->ninterp >= 3
-                                    : noalloc || 2 * n <= 5 * nc);
+        !noalloc && f->precision == ARB_PREC_FP64 && f->table_bytes > kInfinityCache &&
+        f->user_block[0] == 0 && !f->table_loaded &&
+        !(flags & (ARB_Q_TABLE | ARB_Q_SORTED_GLOBAL | ARB_Q_GROUP_ATOMIC)) &&
+        (f->g.ndim == 3 ? f->ninterp >= 3 : 2 * n <= 5 * nc);
     if (automatic) sorted = bucketed_pays(f, n, flags, by_size);
-    // an allocation-free call on a field that queries without a table
-    if (noalloc && by_size) sorted = true;
+    // An allocation-free call on a field that an arb_query has left without a
+    // table: with the table's bits, whatever path is asked for.  Grouped and
+    // on the fly on request and from kCellRows on, where the workspace holds
+    // the rows and buckets, else row by row (k_query_cell).
+    const bool without = noalloc && !f->table && f->tableless && !f->otf;
+    if (without) {
+        flags &= ~(ARB_Q_TABLE | ARB_Q_SORTED_GLOBAL);
+        if (f->BF.nbt == 0) choose_buckets(f, f->BF, false);
+        SortWs w;
+        if (automatic) sorted = n >= kCellRows;
+        sorted &= carve_sort_ws(nullptr, n, f->BF.nbt, false, &w) <=
+                      (int64_t)ARB_NOALLOC_SCRATCH_BYTES &&
+                  (f->g.ndim == 3 ? arb_fused_ok(f->g, f->BF, f->ninterp)
+                                  : arb_fused4_ok(f->g, f->BF));
+    }
     if (n > INT32_MAX - 1) sorted = false;
     if (sorted && f->B.nbt == 0) choose_buckets(f, f->B, true);
     const bool grouped = sorted && !f->table_loaded &&
                          !(flags & (ARB_Q_SORTED_GLOBAL | ARB_Q_GROUP_ATOMIC));
     bool fused = false, fused4 = false;
-    if (grouped && f->g.ndim == 3 && ((flags & ARB_Q_FUSED) || by_size)) {
+    if (grouped && f->g.ndim == 3 && ((flags & ARB_Q_FUSED) || by_size || without)) {
         if (f->BF.nbt == 0) choose_buckets(f, f->BF, false);
         fused = arb_fused_ok(f->g, f->BF, f->ninterp);
     }
-    if (grouped && f->g.ndim == 4 && ((flags & ARB_Q_FUSED) || by_size)) {
+    if (grouped && f->g.ndim == 4 && ((flags & ARB_Q_FUSED) || by_size || without)) {
         if (f->BF.nbt == 0) choose_buckets(f, f->BF, false);
         fused4 = arb_fused4_ok(f->g, f->BF);
     }
@@ -1055,12 +1074,13 @@ static int query_impl(arb_field* f, double* q_dev, int64_t n, int64_t ldq, void*
         if (nodes && !(f->tiles && f->tiles_bytes == arb_tiles_bytes(f->B, f->ninterp, nullptr)))
             return fail(ARB_EINVAL, "%s: the field's node tiles are not allocated; prepare the "
                         "field with one arb_query call with the same flags (n may be 0)", fn);
-        if (!fused && !fused4 && !nodes && !f->table)
+        if (!fused && !fused4 && !nodes && !f->table && !without)
             return fail(ARB_EINVAL, "%s: the field's coefficient table is not allocated; "
                         "prepare the field with arb_build_coeffs", fn);
     }
     if ((fused || fused4) && by_size) f->tableless = 1;
-    int rc = (fused || fused4 || nodes) ? ensure_sentinel(f, s) : arb_build_coeffs(f, stream);
+    int rc = (fused || fused4 || nodes || without) ? ensure_sentinel(f, s)
+                                                   : arb_build_coeffs(f, stream);
     if (rc) return rc;
     if (nodes) {
         rc = ensure_tiles(f, s);
@@ -1087,7 +1107,11 @@ static int query_impl(arb_field* f, double* q_dev, int64_t n, int64_t ldq, void*
     for (float& m : f->last_ms) m = 0.f;
     if (!sorted) {
         if (timing) HIPCHK(hipEventRecord(f->ev[0], s));
-        if (red32)
+        if (without)
+            HIPCHK(arb_launch_query_cell(gq, f->vals, static_cast<const double*>(f->sent),
+                                         f->ninterp, f->has_comps, f->has_norm, q_dev, n, ldq, o,
+                                         s));
+        else if (red32)
             HIPCHK(arb_launch_query_direct_red32(gq, f->precision, out64, f->table, f->ninterp,
                                                  f->has_comps, f->has_norm, q_dev, n, ldq, o,
                                                  s));

@@ -452,6 +452,12 @@ hipError_t arb_launch_query_direct_red32(const ArbGeom& g, int32_t prec, int32_t
                                          const void* table, int32_t ninterp, int32_t has_comps,
                                          int32_t has_norm, const double* q, int64_t n,
                                          int64_t ldq, const ArbOut& o, hipStream_t s);
+// FP64 rows of a field without a table, no workspace (g.red32 as above); sent:
+// the sentinel row.
+hipError_t arb_launch_query_cell(const ArbGeom& g, const double* vals, const double* sent,
+                                 int32_t ninterp, int32_t has_comps, int32_t has_norm,
+                                 const double* q, int64_t n, int64_t ldq, const ArbOut& o,
+                                 hipStream_t s);
 hipError_t arb_launch_query_direct(const ArbGeom& g, int32_t prec, int32_t out_f64,
                                    const void* table, int32_t ninterp, int32_t has_comps,
                                    int32_t has_norm, const double* q, int64_t n, int64_t ldq,

@@ -179,6 +179,8 @@ __device__ __forceinline__ void basis_f32(double loc, double* X, double* dX) {
 template <int D, typename TC>
 __device__ __forceinline__ double contract_basis(const TC* a, const double* const* b) {
     double out = 0.0;
+    // by selects: a runtime index would place the basis in scratch memory
+    const double t0 = b[3][0], t1 = b[3][1], t2 = b[3][2], t3 = b[3][3];
 #pragma unroll 1
     for (int l = 0; l < (D == 4 ? 4 : 1); ++l) {
         double z = 0.0;
@@ -195,9 +197,41 @@ __device__ __forceinline__ double contract_basis(const TC* a, const double* cons
             }
             z = fma(y, b[2][k], z);
         }
-        out = D == 4 ? fma(z, b[3][l], out) : z;
+        out = D == 4 ? fma(z, l < 2 ? (l == 0 ? t0 : t1) : (l == 2 ? t2 : t3), out) : z;
     }
     return out;
+}
+
+// eval_point for g.red32.
+template <int D, typename TC, typename TO>
+__device__ __forceinline__ void eval_point_red32(const TC* a, int32_t has_comps, int32_t has_norm,
+                                                 const double* loc, const ArbGeom& g,
+                                                 const ArbOut& o, int64_t i) {
+    constexpr int K = (D == 3) ? 64 : 256;
+    double X[D][4], dX[D][4];
+#pragma unroll
+    for (int d = 0; d < D; ++d) basis_f32(loc[d], X[d], dX[d]);
+    const double* b[4] = {X[0], X[1], X[2], D == 4 ? X[D - 1] : X[0]};
+    TO rec[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) rec[r] = (TO)0;
+    int k = 0;
+    if (has_comps) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) rec[c] = (TO)contract_basis<D, TC>(a + c * K, b);
+        k = 3;
+    }
+    if (has_norm) {
+        const int r0 = has_comps ? 3 : 0;
+        rec[r0] = (TO)contract_basis<D, TC>(a + k * K, b);
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            const double* bd[4] = {b[0], b[1], b[2], b[3]};
+            bd[d] = dX[d];
+            rec[r0 + 1 + d] = (TO)(contract_basis<D, TC>(a + k * K, bd) / g.h[d]);
+        }
+    }
+    store_rec<D, TO>(rec, has_comps, has_norm, o, i);
 }
 
 template <int D, typename TC, typename TO>
@@ -210,29 +244,98 @@ k_query_direct_red32(ArbGeom g, const TC* __restrict__ table, int32_t ninterp,
     if (i >= n) return;
     double loc[D];
     const int64_t flat = reduce_row<D>(q, ldq, g, o, i, loc);
-    const TC* a = table + flat * (int64_t)ninterp * K;
-    double X[D][4], dX[D][4];
+    eval_point_red32<D, TC, TO>(table + flat * (int64_t)ninterp * K, has_comps, has_norm, loc, g,
+                                o, i);
+}
+
+// ---------------------------------------------------------------------------
+// Rows of an FP64 field that has no table, without grouping and so without a
+// workspace: the allocation-free call's direct path.  A workgroup forms its
+// row's coefficients in LDS with the table build's passes (k_coef.hip) on the
+// cell's 4^D nodes, and one thread evaluates them as the direct kernels do:
+// the table's bits.  For few rows; many are grouped (query_impl's line).
+// ---------------------------------------------------------------------------
+template <int D>
+__global__ void __launch_bounds__(arbs3::SEP_THREADS)
+k_query_cell(ArbGeom g, const double* __restrict__ vals, const double* __restrict__ sent,
+             int32_t ninterp, int32_t has_comps, int32_t has_norm, const double* __restrict__ q,
+             int64_t ldq, ArbOut o) {
+    constexpr int K = (D == 3) ? 64 : 256, NT = D == 4 ? 4 : 1;
+    __shared__ double nodes[NT][64];                // [t][z][y][x], then the powers of t
+    __shared__ __align__(16) double t1[64], t2[64];
+    __shared__ double gc[16], cc[16];
+    __shared__ double a[4 * K];
+    __shared__ double loc[D];
+    __shared__ int64_t cell;
+    const int tid = threadIdx.x;
+    const int64_t i = blockIdx.x;
+    if (tid == 0) {
+        double l[D];
+        cell = reduce_row<D>(q, ldq, g, o, i, l);
 #pragma unroll
-    for (int d = 0; d < D; ++d) basis_f32(loc[d], X[d], dX[d]);
-    const double* b[4] = {X[0], X[1], X[2], D == 4 ? X[D - 1] : X[0]};
-    TO rec[8];
-#pragma unroll
-    for (int r = 0; r < 8; ++r) rec[r] = (TO)0;
-    int k = 0;
-    if (has_comps) {
-        for (int c = 0; c < 3; ++c) rec[c] = (TO)contract_basis<D, TC>(a + c * K, b);
-        k = 3;
+        for (int d = 0; d < D; ++d) loc[d] = l[d];
     }
-    if (has_norm) {
-        const int r0 = has_comps ? 3 : 0;
-        rec[r0] = (TO)contract_basis<D, TC>(a + k * K, b);
+    __syncthreads();
+    if (cell >= g.nc) {                             // the sentinel's row
+        for (int e = tid; e < ninterp * K; e += arbs3::SEP_THREADS) a[e] = sent[e];
+    } else {
+        int64_t src = 0, rem = cell;                // the thread's node: tid = x + 4 y + 16 z + 64 t
+#pragma unroll
         for (int d = 0; d < D; ++d) {
-            const double* bd[4] = {b[0], b[1], b[2], b[3]};
-            bd[d] = dX[d];
-            rec[r0 + 1 + d] = (TO)(contract_basis<D, TC>(a + k * K, bd) / g.h[d]);
+            const int64_t c = d + 1 < D ? rem % g.npos[d] : rem;
+            src += (c + ((tid >> (2 * d)) & 3)) * g.nstride[d];
+            rem /= g.npos[d];
+        }
+        for (int k = 0; k < ninterp; ++k) {
+            __syncthreads();                        // the previous interpolant is done
+            double v = 0.0;
+            if (tid < K) {
+                v = vals[(int64_t)k * g.nnodes + src];
+                (&nodes[0][0])[tid] = v;
+            }
+            const bool bad = __syncthreads_or(!isfinite(v)) != 0;
+            if constexpr (D == 3) {
+                arbs3::sep3_passes<1, 1, 1, false>(nodes[0], t1, t2,
+                                                  [&](int, int, int, int e, double c) {
+                    a[k * K + e] = bad ? (double)NAN : c;
+                });
+            } else {
+                if (tid < 16)                       // corner gx + 2 gy + 4 gz + 8 gt
+                    gc[tid] = arbs4::corner_diff<4, 16, 64>(
+                        &nodes[1 + (tid >> 3)][16 * (1 + ((tid >> 2) & 1)) +
+                                               4 * (1 + ((tid >> 1) & 1)) + 1 + (tid & 1)]);
+                __syncthreads();
+                if (tid < 64) {
+                    double c[4];
+                    arbs3::cub4(nodes[0][tid], nodes[1][tid], nodes[2][tid], nodes[3][tid], c);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) nodes[e][tid] = c[e];
+                } else if (tid < 80) {
+                    const int m = tid - 64;
+                    cc[m] = (m ? gc[m - 1] : 0.0) - gc[m];
+                }
+                __syncthreads();
+                for (int et = 0; et < 4; ++et)
+                    arbs3::sep3_passes4<1, 1, 1, false>(
+                        nodes[et], t1, t2, [&](int, int, int, int exy, const double* c0) {
+                            double c[4] = {c0[0], c0[1], c0[2], c0[3]};
+                            arbs4::shift_rows(cc, exy & 3, exy >> 2, et, c);
+#pragma unroll
+                            for (int ez = 0; ez < 4; ++ez)
+                                a[k * K + exy + 16 * ez + 64 * et] = bad ? (double)NAN : c[ez];
+                        });
+            }
         }
     }
-    store_rec<D, TO>(rec, has_comps, has_norm, o, i);
+    __syncthreads();
+    if (tid != 0) return;
+    double l[D];
+#pragma unroll
+    for (int d = 0; d < D; ++d) l[d] = loc[d];
+    if (g.red32)
+        eval_point_red32<D, double, double>(a, has_comps, has_norm, l, g, o, i);
+    else
+        eval_point<D, double, double, double>(a, has_comps, has_norm, l, g, o, i);
 }
 
 // ---------------------------------------------------------------------------
@@ -2137,6 +2240,22 @@ hipError_t arb_launch_query_direct_red32(const ArbGeom& g, int32_t prec, int32_t
                                       n, ldq, o, s);
     return launch_direct_red32<4>(g, prec, out_f64, table, ninterp, has_comps, has_norm, q, n,
                                   ldq, o, s);
+}
+
+hipError_t arb_launch_query_cell(const ArbGeom& g, const double* vals, const double* sent,
+                                 int32_t ninterp, int32_t has_comps, int32_t has_norm,
+                                 const double* q, int64_t n, int64_t ldq, const ArbOut& o,
+                                 hipStream_t s) {
+    if (n <= 0) return hipSuccess;
+    if (n > INT32_MAX) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)n), block(arbs3::SEP_THREADS);
+    if (g.ndim == 3)
+        hipLaunchKernelGGL(k_query_cell<3>, grid, block, 0, s, g, vals, sent, ninterp, has_comps,
+                           has_norm, q, ldq, o);
+    else
+        hipLaunchKernelGGL(k_query_cell<4>, grid, block, 0, s, g, vals, sent, ninterp, has_comps,
+                           has_norm, q, ldq, o);
+    return hipGetLastError();
 }
 
 hipError_t arb_launch_query_direct(const ArbGeom& g, int32_t prec, int32_t out_f64,

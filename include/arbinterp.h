@@ -223,7 +223,9 @@ int arb_query(arb_field* f, double* q_dev, int64_t n, int64_t ldq,
  *     arb_build_coeffs) or node tiles (mixed 3D: one arb_query with the same
  *     flags, n may be 0); they are rebuilt in place after
  *     arb_field_set_values.  A large FP64 field that an arb_query has answered
- *     without a table needs neither.  Otherwise ARB_EINVAL;
+ *     without a table needs neither: its coefficients are formed on the fly,
+ *     with the table's bits, whichever path the flags ask for (ARB_Q_TABLE
+ *     included; small calls are faster with the table).  Otherwise ARB_EINVAL;
  *   - n <= ARB_NOALLOC_MAX_ROWS, and the workspace of n rows over the field's
  *     buckets must fit the array (about 16 bytes per row, 32 on the mixed 3D
  *     node-tile path, plus 8 per bucket), else ARB_EINVAL with the sizes in
