@@ -29,36 +29,40 @@ __device__ __forceinline__ unsigned long long mix64(unsigned long long x) {
     return x;
 }
 
-// Insert key into the device-wide set of `axis`; a new one is listed.
-__device__ void axis_insert(const AxesLayout& L, int axis, unsigned long long key) {
+// Insert key into the device-wide set of `axis`; a new one is listed.  False
+// where the set cannot take it (overflow: more than AXES_MAX values).  Up to
+// AXES_MAX keys fill half of the slots, in runs of some 50 at most; but every
+// thread that has read the count before the others raised it may add one, and
+// rows that form no grid can fill the set: a run past AXES_PROBES is an
+// overflow, as is an empty slot with the count used up.
+constexpr int AXES_PROBES = 256;
+
+__device__ bool axis_insert(const AxesLayout& L, int axis, unsigned long long key) {
     unsigned long long* tab = L.hash + (int64_t)axis * AXES_SLOTS;
     unsigned int slot = (unsigned int)mix64(key) & (AXES_SLOTS - 1);
-    // at most AXES_MAX keys and the few inserted while the count is read: an
-    // empty slot or the key is always reached
-    for (int probe = 0; probe < AXES_SLOTS; ++probe) {
+    for (int probe = 0; probe < AXES_PROBES; ++probe) {
         const unsigned long long cur = __hip_atomic_load(&tab[slot], __ATOMIC_RELAXED,
                                                          __HIP_MEMORY_SCOPE_AGENT);
-        if (cur == key) return;
+        if (cur == key) return true;
         if (cur == kEmpty) {
             if (__hip_atomic_load(&L.head->count[axis], __ATOMIC_RELAXED,
-                                  __HIP_MEMORY_SCOPE_AGENT) >= AXES_MAX) {
-                L.head->overflow = 1;
-                return;
-            }
+                                  __HIP_MEMORY_SCOPE_AGENT) >= AXES_MAX)
+                break;
             const unsigned long long old = atomicCAS(&tab[slot], kEmpty, key);
-            if (old == key) return;
+            if (old == key) return true;
             if (old == kEmpty) {
                 const unsigned int p = atomicAdd(&L.head->count[axis], 1u);
                 const double x = __longlong_as_double((long long)key);
                 if (p < AXES_FEW) L.few[axis * AXES_FEW + p] = x;
                 else if (p < AXES_MAX) L.more[(int64_t)axis * AXES_MAX + p - AXES_FEW] = x;
-                else L.head->overflow = 1;
-                return;
+                else break;
+                return true;
             }
         }
         slot = (slot + 1) & (AXES_SLOTS - 1);
     }
     L.head->overflow = 1;
+    return false;
 }
 
 // The values a workgroup has met, per axis: LDS_SLOTS slots, LDS_PROBES tried;
@@ -71,7 +75,9 @@ k_axes(const double* __restrict__ rows, int64_t nrows, int64_t ld, AxesLayout L)
     __shared__ unsigned long long met[D][LDS_SLOTS];
     for (int i = threadIdx.x; i < D * LDS_SLOTS; i += 256) (&met[0][0])[i] = kEmpty;
     __syncthreads();
-    bool bad = false;
+    // bad, over: a non-finite coordinate, an overflow of the sets (their lists are
+    // then not used, and only the coordinates are looked at)
+    bool bad = false, over = false;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nrows;
          i += (int64_t)gridDim.x * 256) {
         double x[D];
@@ -80,7 +86,7 @@ k_axes(const double* __restrict__ rows, int64_t nrows, int64_t ld, AxesLayout L)
             x[a] = rows[i * ld + a] + 0.0;          // -0.0 -> +0.0
             bad |= !isfinite(x[a]);
         }
-        if (bad) continue;
+        if (bad || over) continue;
 #pragma unroll
         for (int a = 0; a < D; ++a) {
             const unsigned long long key = (unsigned long long)__double_as_longlong(x[a]);
@@ -100,7 +106,7 @@ k_axes(const double* __restrict__ rows, int64_t nrows, int64_t ld, AxesLayout L)
                 }
                 slot = (slot + 1) & (LDS_SLOTS - 1);
             }
-            if (ask) axis_insert(L, a, key);
+            if (ask && !axis_insert(L, a, key)) over = true;
         }
     }
     if (bad) L.head->nonfinite = 1;
