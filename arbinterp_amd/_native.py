@@ -94,6 +94,7 @@ SIGNATURES = [
     ("arb_csv_shape", c_i32, [ctypes.c_char_p, ctypes.POINTER(c_i64), ctypes.POINTER(c_i32)]),
     ("arb_csv_read", c_i32, [ctypes.c_char_p, c_vp, c_i64, c_i32]),
     ("arb_field_destroy", None, [c_vp]),
+    ("arb_release_memory", c_i64, []),
     ("arb_last_error", ctypes.c_char_p, []),
     ("arb_version", ctypes.c_char_p, []),
 ]

@@ -46,7 +46,8 @@ static int fail(int code, const char* fmt, ...) {
 // queries, hipFree alone took 1.3 of 1.9 ms.  Larger blocks (tables), and what
 // a living field gives up, are freed at once.  A block enters the pool when
 // nothing uses it any more (as hipFree waits for that), so whatever thread or
-// stream takes it next may write it.
+// stream takes it next may write it.  arb_release_memory empties it, for other
+// allocators on the device.
 // ---------------------------------------------------------------------------
 namespace {
 
@@ -119,6 +120,13 @@ struct DevPool {
             return hipFree(b.p);
         }
         return hipSuccess;
+    }
+
+    int64_t release() {
+        std::lock_guard<std::mutex> lock(mu);
+        const size_t was = held;
+        shrink(0);
+        return (int64_t)was;
     }
 
     void shrink(size_t most) {                       // (with mu held)
@@ -1798,6 +1806,8 @@ int arb_table_load(arb_field* f, int64_t cell0, int64_t ncells, const void* src_
     f->table_loaded = 1;      // the table is authoritative: queries read it
     return ARB_OK;
 }
+
+int64_t arb_release_memory(void) { return dev_pool().release(); }
 
 void arb_field_destroy(arb_field* f) {
     if (!f) return;

@@ -370,8 +370,14 @@ int arb_operator_matrix(int32_t ndim, int32_t which, double* out);
 int arb_csv_shape(const char* path, int64_t* nrows, int32_t* ncols);
 int arb_csv_read(const char* path, double* out, int64_t nrows, int32_t ncols);
 
-/* Release the handle and its device memory. */
+/* Release the handle and its device memory.  Up to 512 MB of what destroyed
+ * fields held is kept for the process's next fields (it is also given back
+ * when an allocation of theirs fails). */
 void arb_field_destroy(arb_field* f);
+
+/* Give the device memory kept from destroyed fields back to the device, for
+ * other allocators.  Returns its bytes.  Any thread may call it. */
+int64_t arb_release_memory(void);
 
 /* Thread-local message for the last failing call on this thread. */
 const char* arb_last_error(void);
