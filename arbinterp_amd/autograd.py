@@ -46,9 +46,11 @@ class InterpFunction(torch.autograd.Function):
         N.check(N.lib().arb_field_set_values(interp._h, _ptr(vals), _stream_handle(torch)),
                 "set_values")
         interp._info.table_built = 0
-        # forward and backward read the same coefficient source: node tiles
-        # for mixed 3D fields (an FP64 model per block plus FP32 residuals;
-        # no table is built), the table otherwise; one build per set of values
+        # forward and backward evaluate the same coefficients: node tiles for
+        # mixed 3D fields (an FP64 model per block plus FP32 residuals; no
+        # table is built); otherwise the table's, which the forward of a large
+        # FP64 field forms on the fly and the backward builds, once per set of
+        # values
         _, U, G = interp.query_device(q, out_f64=True)
         ctx.save_for_backward(q)
         ctx.interp = interp

@@ -930,9 +930,12 @@ static int ensure_group(arb_field* f, int64_t n) {
 // (which touch fewer cells) from 0.5: the line lies where neither loses to the
 // former one.  That was 65536 rows and one per two cells, per four with node
 // tiles: 2.5e5 rows of the small 3D grid and one interpolant took 92 us for
-// 30, 1e6 rows of the large one 289 for 126.  A field that queries without its
-// table (by_size) and has none is taken from there on: the direct kernel would
-// build it first.
+// 30, 1e6 rows of the large one 289 for 126.  In 3D, a field that queries
+// without its table (by_size) and has none is taken from there on: the direct
+// kernel would build it first.  (Not in 4D: over and over at 0.5 to 0.75 rows
+// per cell the direct kernel is the faster one, 249 us for 397 with three
+// interpolants of 40 x 37 x 30 x 12 nodes, and no table was built for less
+// before either.)
 static bool bucketed_pays(arb_field* f, int64_t n, int32_t flags, bool by_size) {
     const int64_t nc = f->g.nc;
     const bool mixed = f->precision == ARB_PREC_MIXED, one = f->ninterp == 1;
@@ -1013,6 +1016,15 @@ static int query_impl(arb_field* f, double* q_dev, int64_t n, int64_t ldq, void*
     // rows in a cloud 0.28 / 0.27; 40 x 37 x 30 x 12 nodes, 6.5 rows per cell:
     // four interpolants 0.92 / 1.18, but in a cloud 0.76 / 0.45, and one
     // interpolant 0.29 / 0.20.  FP32 tables are half the bytes: 0.45 / 0.30.
+    // Rows in a cloud touch few cells, whose part of a table stays cached.  When
+    // they come over and over, the table is the faster one for most fields
+    // (whole call, us, this / the table's, Gaussian of 0.08 of the box): 'both'
+    // on 112 x 96 x 88, one row per cell of the field 229 / 212, five 654 / 516;
+    // on 128^3 535 / 617 and 1545 / 1505; 40 x 37 x 30 x 12 at 1.5 rows per cell,
+    // one interpolant 167 / 137, four 336 / 280 (uniform 532 / 1225).  The line
+    // does not know the spread: it lies where the larger ratio is on this
+    // side, and a table costs some 30 ms per GB before its first use.
+    // ARB_Q_TABLE, or the autotuner on the caller's positions, has it.
     constexpr int64_t kInfinityCache = (int64_t)256 << 20;
     const int64_t nc = f->g.nc;
     const bool by_size =

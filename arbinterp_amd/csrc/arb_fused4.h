@@ -1,8 +1,8 @@
 // Quadcubic coefficients of a block of 4 x 4 x 2 cells in (x, y, z) at one
-// t, formed in LDS from node values, for the kernels that evaluate without
-// the coefficient table: the 4D query (k_query.hip) and the 4D backward
-// (k_backward.hip).  The operations of the table build (k_coef.hip,
-// arb_sep4.h) in its order, so the coefficients are the table's bits.
+// t, formed in LDS from node values, for the 4D query that evaluates without
+// the coefficient table (k_query.hip).  The operations of the table build
+// (k_coef.hip, arb_sep4.h) in its order, so the coefficients are the table's
+// bits.
 //
 // A row takes four lanes, one per power et of t.  passes() leaves in LDS, for
 // every et, the 16 (ex, ey) values of each (cell column, node plane) after

