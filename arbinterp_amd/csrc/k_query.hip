@@ -968,7 +968,8 @@ k_eval_bucket(ArbGeom g, ArbBuckets B, const TC* __restrict__ table, int32_t has
 //
 // 128^3 FP64 'both', 10^7 rows: 0.94 ms, against 1.33 ms for the staged table
 // kernel (4 GB of coefficients through HBM; here 0.35 GB of nodes); 112 x 96 x
-// 88, 10^6 rows: 0.265 against 0.38 ms.  VALU issue (0.45 ms of the first) and
+// 88, 10^6 rows: 0.265 against 0.38 ms.  VALU issue (0.45 ms of the first,
+// profiles/eval_fused_fp64_dipole3d_counters.txt) and
 // the chain row index -> position -> sort ahead of the passes bound it, at four
 // waves per SIMD (at three: 0.30 ms for the second).  The same kernel with
 // the coefficients of one interpolant at a time in LDS took 1.27 ms (LDS
@@ -1291,8 +1292,9 @@ k_eval_fused3(ArbGeom g, ArbBuckets B, const double* __restrict__ vals,
 //
 // 48^3 x 16 nodes, FP64, one interpolant, 2e6 rows (1.7 per cell): 0.46 ms,
 // against 0.71 ms for the staged table kernel, which reads 2.4 GB (and whose
-// table takes 0.53 ms to build); 6e5 rows 0.40 against 0.67 ms.  About 0.2 ms
-// of it is VALU issue and 0.18 ms LDS; the rest is what two waves per SIMD
+// table takes 0.53 ms to build); 6e5 rows 0.40 against 0.67 ms.  About 0.22 ms
+// of it is VALU issue and 0.20 ms LDS
+// (profiles/eval_fused4_moving4d_counters.txt); the rest is what two waves per SIMD
 // leave of the barriers between the passes.  Measured without gain: one layer
 // per workgroup (0.75 ms: the chain bounds -> row index -> position and the
 // node loads), rows put in cell order first (0.49 ms: LDS conflicts fall from

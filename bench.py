@@ -69,7 +69,8 @@ def parse():
                     help="only the headline path (default flags, output arrays): --steps "
                          "queries (for counter runs; no oracle, no CPU baseline, no JSON line)")
     ap.add_argument("--precision", choices=["mixed", "fp64"], default="mixed",
-                    help="field precision of --profile-only (fp64: the FP64 table path)")
+                    help="field precision of --profile-only (fp64: the default FP64 path; with "
+                         "--flags 2048 its table path)")
     return ap.parse_args()
 
 
@@ -159,6 +160,9 @@ def main():
     res = {}
     for prec in ("mixed", "fp64"):
         t = tricubic(rows, "quiet", mode="both", precision=prec)
+        # whether the default path holds a table (a large FP64 field does not)
+        t.query_device(qd)
+        reads_table = bool(t.field_info().table_built)
         build_ms = one_off_build_ms(torch, t, qd)
         # output layouts: "arrays" the reference's three arrays (comps N x 3,
         # |B| N, grad N x 3; FP32 for mixed, FP64 for fp64: the drop-in's
@@ -206,7 +210,8 @@ def main():
             host = {"ms_per_call": hms, "queries_per_s": args.nq / hms * 1e3,
                     "calls": args.host_calls}
             log("host numpy Query: %.2f ms per call" % hms)
-        res[prec] = dict(obj=t, build_ms=build_ms, out=out, per=per, host=host)
+        res[prec] = dict(obj=t, build_ms=build_ms, out=out, per=per, host=host,
+                         reads_table=reads_table)
     nc = res["mixed"]["obj"].nc
     cells = res["mixed"]["out"][3]
     valid = cells[cells < nc]
@@ -250,14 +255,19 @@ def main():
     # reference's output layout.  roofline.achieved: the algorithmic bytes of
     # the evaluation (N*(24 + 7*s_o) + U*4*64*s_c: FP64 positions in, 7 outputs,
     # each touched cell's 4 x 64 coefficients once; FP32 s_o = s_c = 4 for the
-    # mixed path) over the evaluation kernel's own HIP-event duration.
+    # mixed path) over the evaluation kernel's own HIP-event duration.  The FP64
+    # path is priced by the source of coefficients it reads: the table's touched
+    # cells, or each node value once where it forms them on the fly.
     N = args.nq
     ms = res["mixed"]["per"]["auto"]["ms_per_step"]
     ms64 = res["fp64"]["per"]["auto"]["ms_per_step"]
     st = res["mixed"]["per"]["auto"]["stage_ms"]
     st64 = res["fp64"]["per"]["auto"]["stage_ms"]
     alg_bytes = N * (24 + 7 * 4) + U * 4 * 64 * 4
-    alg64 = N * (24 + 7 * 8) + U * 4 * 64 * 8
+    rows64 = N * (24 + 7 * 8)
+    table64 = rows64 + U * 4 * 64 * 8
+    on_table = res["fp64"]["reads_table"]
+    alg64 = table64 if on_table else rows64 + int(res["fp64"]["obj"].field_info().nnodes) * 4 * 8
     node_bytes = N * (16 + 4 + 32) + UB * tile_bytes   # row record, row index, output record
     ev_ms = st[3] or ms
     ev64 = st64[3] or ms64
@@ -286,6 +296,8 @@ def main():
 
     per_m = res["mixed"]["per"]
     per_d = res["fp64"]["per"]
+    tab = per_d.get("sorted_table")
+    tab_ev = tab and tab["stage_ms"][3]
     qps = N / (ms * 1e-3)
     line = {
         "metric": METRIC,
@@ -332,9 +344,16 @@ def main():
                      "within_bound": within, "sample_rows": int(len(idx))},
         "fp64_plain": {"value": N / (ms64 * 1e-3), "ms_per_step": ms64,
                        "eval_kernel_ms": ev64, "split_ms": st64[4],
+                       "coefficients": "table" if on_table else "formed from node values",
                        "roofline_achieved_GBs": ach64, "frac": ach64 / HBM_PEAK_GBS,
-                       "algorithmic_bytes": alg64},
+                       "algorithmic_bytes": alg64,
+                       "table_path": tab and {
+                           "ms_per_step": tab["ms_per_step"], "eval_kernel_ms": tab_ev,
+                           "algorithmic_bytes": table64,
+                           "roofline_achieved_GBs": table64 / (tab_ev * 1e-3) / 1e9,
+                           "frac": table64 / (tab_ev * 1e-3) / 1e9 / HBM_PEAK_GBS}},
         "speedup_vs_fp64": ms64 / ms,
+        "speedup_vs_fp64_table": tab and tab["ms_per_step"] / ms,
         "packed_records": {
             "mixed_p64_ms": per_m["auto_p64"]["ms_per_step"],
             "mixed_p32_ms": per_m["auto_p32"]["ms_per_step"],
